@@ -45,6 +45,15 @@ enum { TSMI_F32 = 0, TSMI_F16 = 1, TSMI_BF16 = 2 };
  * (std::invalid_argument -> ValueError, std::runtime_error -> RuntimeError). */
 const char *tsmi_last_error(void);
 
+/* Voxels of a point cloud in host memory: cell = floor(coordinate / voxel) in double per axis, the
+ * distinct cells in ascending (x, y, z) order (voxels int32 [m, 3]), the first point of each (index
+ * int64 [m]) and the voxel of every point (inverse int64 [n]); utils/quantize.py:10-54.  kind: 0 float,
+ * 1 double, 2 int32, 3 int64; rows and columns are row_bytes / col_bytes apart; voxels and index have
+ * room for n; index and inverse may be NULL.  *n_voxels = m, or -1 when a cell does not fit int32 or
+ * cells and points together do not fit 64 bits (nothing is then written that counts). */
+int tsmi_host_voxelize(const void *points, int kind, int64_t n, int64_t row_bytes, int64_t col_bytes,
+                       const double *voxel, int32_t *voxels, int64_t *index, int64_t *inverse, int64_t *n_voxels);
+
 /* ABI version of the library (bumped on any signature change). */
 int tsmi_version(void);
 

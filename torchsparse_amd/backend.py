@@ -61,6 +61,7 @@ def _load():
     lib.tsmi_kmap_sorted_samples_elems.restype = _i64
     lib.tsmi_kmap_sorted_samples_elems.argtypes = [_i64]
     sig = {
+        "tsmi_host_voxelize": [_vp, _i32, _i64, _i64, _i64, _vp, _vp, _vp, _vp, _vp],
         "tsmi_hashtable_clear": [_vp, _vp, _vp, _i64],
         "tsmi_hashtable_insert_coords": [_vp, _vp, _vp, _i64, _vp, _i64, _vp],
         "tsmi_hashtable_insert_keys": [_vp, _vp, _vp, _i64, _vp, _i64, _vp],
@@ -154,7 +155,8 @@ class _Library:
     the entry points that only answer a question are passed through as they are."""
 
     _ASIS = ("tsmi_conv_implicit_gemm_packed", "tsmi_conv_implicit_gemm_segments_packed",
-             "tsmi_conv_implicit_gemm_grouped_packed", "tsmi_last_error", "tsmi_version")
+             "tsmi_conv_implicit_gemm_grouped_packed", "tsmi_last_error", "tsmi_version",
+             "tsmi_host_voxelize")
     _ASIS_ENDINGS = ("_elems", "_supported", "_bytes", "_capacity", "_padded")
 
     def __init__(self, lib):
@@ -2778,6 +2780,35 @@ def conv_forward_gather_scatter_cuda(in_feats, kernel, nbmaps, nbsizes, input_ma
 
 
 # ------------------------------------------------------------ point-voxel operators
+
+
+_HOST_KINDS = {"float32": 0, "float64": 1, "int32": 2, "int64": 3}
+
+
+def host_voxelize(coords, voxel_size, want_index: bool, want_inverse: bool):
+    """(voxels int32 [M, 3], index int64 [M] or None, inverse int64 [N] or None) of host points
+    [N, 3] (a numpy array, any strides): tsmi_host_voxelize.  None for what that call does not take:
+    other shapes and types, no points, a division that is not one of doubles, cells outside int32."""
+    import numpy as np
+    kind = _HOST_KINDS.get(coords.dtype.name)
+    voxel = np.asarray(voxel_size)
+    if (kind is None or coords.ndim != 2 or coords.shape[1] != 3 or coords.shape[0] == 0
+            or not coords.dtype.isnative or voxel.dtype.name not in ("float64", "int64")):
+        return None
+    n = coords.shape[0]
+    voxel = np.ascontiguousarray(voxel, dtype=np.float64)
+    voxels = np.empty((n, 3), dtype=np.int32)
+    index = np.empty(n, dtype=np.int64) if want_index else None
+    inverse = np.empty(n, dtype=np.int64) if want_inverse else None
+    count = ctypes.c_int64()
+    _check(_C.tsmi_host_voxelize(coords.ctypes.data, kind, n, coords.strides[0], coords.strides[1],
+                                 voxel.ctypes.data, voxels.ctypes.data, index.ctypes.data if want_index else None,
+                                 inverse.ctypes.data if want_inverse else None, ctypes.byref(count)))
+    m = count.value
+    if m < 0:
+        return None
+    # (rows that were not needed were never written: the views hold on to addresses, not to memory)
+    return voxels[:m], index[:m] if want_index else None, inverse
 
 
 def hash_cuda(coords: torch.Tensor) -> torch.Tensor:

@@ -21,7 +21,7 @@ def _as_tensor(v):
 def sparse_collate(inputs: List[SparseTensor]) -> SparseTensor:
     stride = inputs[0].stride
     rows, feats = [], []
-    for b, sample in enumerate(inputs):
+    for sample in inputs:
         sample.coords, sample.feats = _as_tensor(sample.coords), _as_tensor(sample.feats)
         if not isinstance(sample.coords, torch.Tensor):
             raise AssertionError(type(sample.coords))
@@ -29,10 +29,23 @@ def sparse_collate(inputs: List[SparseTensor]) -> SparseTensor:
             raise AssertionError(type(sample.feats))
         if sample.stride != stride:
             raise AssertionError((sample.stride, stride))
-        c = sample.coords
-        rows.append(torch.cat((c.new_full((c.shape[0], 1), b, dtype=torch.int), c), dim=1))
+        rows.append(sample.coords)
         feats.append(sample.feats)
-    return SparseTensor(coords=torch.cat(rows, dim=0), feats=torch.cat(feats, dim=0), stride=stride)
+    first = rows[0]
+    if all(c.dtype == torch.int32 and c.device == first.device and c.dim() == 2 and c.shape[1] == first.shape[1]
+           for c in rows):
+        # every row is written once, where it stays
+        coords = first.new_empty((sum(c.shape[0] for c in rows), first.shape[1] + 1))
+        at = 0
+        for b, c in enumerate(rows):
+            part = coords[at:at + c.shape[0]]
+            part[:, 0] = b
+            part[:, 1:] = c
+            at += c.shape[0]
+    else:
+        coords = torch.cat([torch.cat((c.new_full((c.shape[0], 1), b, dtype=torch.int), c), dim=1)
+                            for b, c in enumerate(rows)], dim=0)
+    return SparseTensor(coords=coords, feats=torch.cat(feats, dim=0), stride=stride)
 
 
 def sparse_collate_fn(inputs: List[Any]) -> Any:

@@ -31,6 +31,13 @@ def sparse_quantize(coords, voxel_size: Union[float, Tuple[float, ...]] = 1, *,
         voxel_size = (voxel_size,) * 3
     if not (isinstance(voxel_size, tuple) and len(voxel_size) == 3):
         raise AssertionError(voxel_size)
+    coords = np.asarray(coords)
+    from .. import backend
+    native = backend.host_voxelize(coords, voxel_size, return_index, return_inverse)
+    if native is not None:
+        out = [part for part in native if part is not None]
+        return out[0] if len(out) == 1 else out
+    # (points the native call does not take)
     voxels = np.floor(np.asarray(coords) / np.asarray(voxel_size)).astype(np.int32)
     _, index, inverse = np.unique(ravel_hash(voxels), return_index=True, return_inverse=True)
     out = [voxels[index]]
