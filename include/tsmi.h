@@ -680,6 +680,22 @@ int tsmi_hash_coords(tsmi_stream_t s, const int32_t *coords, int64_t n, int64_t 
 int tsmi_kernel_hash(tsmi_stream_t s, const int32_t *coords, int64_t n, const int32_t *offsets,
                      int kvol, int64_t *out);
 
+/* An index over n 64-bit keys (references of sphashquery) in device memory, int32 `index` of
+ * tsmi_hash_index_words(n) words (-1: 2^29 keys or more), and its look-ups: out[i] = a row r with keys[r] == queries[i], or -1.  The keys themselves are read by
+ * the look-ups and must stay as they were. */
+int64_t tsmi_hash_index_words(int64_t n);
+int tsmi_hash_index_build(tsmi_stream_t s, const int64_t *keys, int64_t n, int32_t *index);
+int tsmi_hash_index_find(tsmi_stream_t s, const int64_t *keys, int64_t n, const int32_t *index,
+                         const int64_t *queries, int64_t m, int32_t *out);
+
+/* weights float [n, 8]: trilinear weights of points (float, rows row_stride and columns col_stride
+ * elements apart) with respect to the corners of their cell of edge `scale`, x slowest, low before high;
+ * a corner whose index (int32 or, index64, int64; strides in elements) is -1 has none, and the rest sum
+ * to one (nn/functional/devoxelize.py:11-48 of the reference). */
+int tsmi_ti_weights(tsmi_stream_t s, const float *points, int64_t n, int64_t row_stride, int64_t col_stride,
+                    const void *index, int index64, int64_t index_row_stride, int64_t index_col_stride,
+                    float scale, float *weights);
+
 /* out[v] = number of i with idx[i] == v for v in [0, num); other indices are skipped.  `out`
  * is cleared here.  Replaces count_cuda (others/count_cuda.cu:10-31). */
 int tsmi_count(tsmi_stream_t s, const int32_t *idx, int64_t n, int32_t *out, int num);
@@ -687,8 +703,8 @@ int tsmi_count(tsmi_stream_t s, const int32_t *idx, int64_t n, int32_t *out, int
 /* Grouping of an index array, the preparation of the two row sums below: `order` int32[m]
  * receives the positions e of idx with 0 <= idx[e] < n_groups sorted by (idx[e], e) — only the
  * first starts[n_groups] entries are meaningful — and starts int32[n_groups + 1] the beginning of
- * every group's run.  `temp` holds tsmi_group_temp_bytes(m) bytes.  A radix sort over the bits
- * n_groups needs plus one binary search per group; no host read-back.  No counterpart in the
+ * every group's run.  `temp` holds tsmi_group_temp_bytes(m) bytes.  A stable two-level sort over
+ * the bits n_groups needs, four launches (more than 2^21 groups: a library sort); no host read-back.  No counterpart in the
  * reference, which adds with atomicAdd instead. */
 int64_t tsmi_group_temp_bytes(int64_t m);
 int tsmi_group_by_index(tsmi_stream_t s, const int32_t *idx, int64_t m, int64_t n_groups, void *temp,

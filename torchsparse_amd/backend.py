@@ -52,6 +52,8 @@ def _load():
     lib.tsmi_conv_workspace_elems.argtypes = [_i64, _i64, _i32, _i32, _i32, _i32, _i32, _i32]
     lib.tsmi_group_temp_bytes.restype = _i64
     lib.tsmi_group_temp_bytes.argtypes = [_i64]
+    lib.tsmi_hash_index_words.restype = _i64
+    lib.tsmi_hash_index_words.argtypes = [_i64]
     lib.tsmi_wgrad_pairs_capacity.restype = _i64
     lib.tsmi_wgrad_pairs_capacity.argtypes = [_i64, _i32]
     lib.tsmi_conv_wgrad_pairs_workspace_elems.restype = _i64
@@ -124,6 +126,9 @@ def _load():
         "tsmi_map_group_rows": [_vp, _vp, _i64, _i32, _i32, _vp, _vp, _vp, _vp, _vp],
         "tsmi_hash_coords": [_vp, _vp, _i64, _vp],
         "tsmi_kernel_hash": [_vp, _vp, _i64, _vp, _i32, _vp],
+        "tsmi_hash_index_build": [_vp, _vp, _i64, _vp],
+        "tsmi_hash_index_find": [_vp, _vp, _i64, _vp, _vp, _i64, _vp],
+        "tsmi_ti_weights": [_vp, _vp, _i64, _i64, _i64, _vp, _i32, _i64, _i64, _f32, _vp],
         "tsmi_count": [_vp, _vp, _i64, _vp, _i32],
         "tsmi_group_by_index": [_vp, _vp, _i64, _i64, _vp, _i64, _vp, _vp],
         "tsmi_voxelize_forward": [_vp, _vp, _vp, _vp, _vp, _i64, _i32, _i64, _i32, _vp],
@@ -157,7 +162,7 @@ class _Library:
     _ASIS = ("tsmi_conv_implicit_gemm_packed", "tsmi_conv_implicit_gemm_segments_packed",
              "tsmi_conv_implicit_gemm_grouped_packed", "tsmi_last_error", "tsmi_version",
              "tsmi_host_voxelize")
-    _ASIS_ENDINGS = ("_elems", "_supported", "_bytes", "_capacity", "_padded")
+    _ASIS_ENDINGS = ("_elems", "_words", "_supported", "_bytes", "_capacity", "_padded")
 
     def __init__(self, lib):
         self._lib = lib
@@ -2826,6 +2831,42 @@ def kernel_hash_cuda(coords: torch.Tensor, kernel_offset: torch.Tensor) -> torch
     out = torch.empty((offsets.shape[0], coords.shape[0]), dtype=torch.int64, device=coords.device)
     _check(_C.tsmi_kernel_hash(_stream(), _ptr(coords), coords.shape[0], _ptr(offsets),
                                offsets.shape[0], _ptr(out)))
+    return out
+
+
+def hash_query(queries: torch.Tensor, references: torch.Tensor) -> torch.Tensor:
+    """int32 [n]: for every int64 query a row of ``references`` (contiguous int64 [m]) that holds it, or
+    -1.  The index over the references is kept on their tensor (and rebuilt when it is modified in
+    place): a point-voxel network asks for its points, and again for the corners of their cells, against
+    the hashes of one voxel set."""
+    queries, references = _need(queries, torch.int64, "queries"), _need(references, torch.int64, "references")
+    n, stream = references.numel(), _stream()
+    keep = not references.is_inference()  # (an inference tensor has no version to go by)
+    cached = getattr(references, "_tsmi_index", None) if keep else None
+    if (cached is not None and cached[0] == references._version and cached[1] == references.data_ptr()
+            and cached[2] == stream):
+        index = cached[3]
+    else:
+        index = torch.empty(_C.tsmi_hash_index_words(n), dtype=torch.int32, device=references.device)
+        _check(_C.tsmi_hash_index_build(stream, references.data_ptr(), n, index.data_ptr()))
+        if keep:
+            references._tsmi_index = (references._version, references.data_ptr(), stream, index)
+    out = torch.empty(queries.numel(), dtype=torch.int32, device=queries.device)
+    _check(_C.tsmi_hash_index_find(stream, references.data_ptr(), n, index.data_ptr(), queries.data_ptr(),
+                                   queries.numel(), out.data_ptr()))
+    return out
+
+
+def ti_weights_cuda(coords: torch.Tensor, idx_query: torch.Tensor, scale: float) -> Optional[torch.Tensor]:
+    """float [N, 8] trilinear weights of float32 GPU points [N, 3] (tsmi_ti_weights); None for operands
+    of other kinds."""
+    if not (coords.is_cuda and idx_query.is_cuda and coords.dtype == torch.float32 and coords.dim() == 2
+            and coords.shape[1] == 3 and idx_query.dim() == 2 and idx_query.shape == (coords.shape[0], 8)
+            and idx_query.dtype in (torch.int32, torch.int64) and coords.device == idx_query.device):
+        return None
+    out = torch.empty((coords.shape[0], 8), dtype=torch.float32, device=coords.device)
+    _check(_C.tsmi_ti_weights(_stream(), coords.data_ptr(), coords.shape[0], *coords.stride(), idx_query.data_ptr(),
+                              int(idx_query.dtype == torch.int64), *idx_query.stride(), float(scale), out.data_ptr()))
     return out
 
 

@@ -13,6 +13,9 @@ def calc_ti_weights(coords: torch.Tensor, idx_query: torch.Tensor, scale: float 
     of their cell of edge ``scale`` (corner order: x slowest, z fastest, low before high);
     corners that do not exist (idx_query == -1) get weight 0 and the rest is renormalised."""
     with torch.no_grad():
+        w = backend.ti_weights_cuda(coords, idx_query, scale)
+        if w is not None:
+            return w
         p = coords
         low = torch.floor(p / scale) * scale if scale != 1 else torch.floor(p)
         frac_hi = (p - low).float()            # distance to the low corner, per axis
