@@ -397,6 +397,9 @@ int64_t tsmi_packed_weight_elems(int kvol, int cin, int cout);
  * No counterpart in the reference (its kernels read [K_vol,Cin,Cout] directly). */
 int tsmi_pack_weights(tsmi_stream_t s, const void *w, void *w_packed, int kvol, int cin,
                       int cout, int dtype);
+/* The same for n tensors of one type in one launch (48 at a time); shapes: n rows (K_vol, Cin, Cout). */
+int tsmi_pack_weights_many(tsmi_stream_t s, const void *const *w, void *const *w_packed,
+                           const int32_t *shapes, int n, int dtype);
 
 /* Floats of scratch the implicit-GEMM entry points want for a problem of
  * n_tile_rows map rows (n_out for the unsorted call, n_pad and sorted = 1 for the
@@ -507,6 +510,10 @@ int64_t tsmi_conv_wgrad_pairs_workspace_elems(int64_t pair_cap, int kvol, int ci
 int tsmi_conv_wgrad_pairs(tsmi_stream_t s, const void *x, const void *dy, const int32_t *pairs,
                           const int32_t *seg_steps, int64_t pair_cap, int x_col, int kvol, int cin,
                           int cout, int dtype, float *workspace, int64_t workspace_elems, void *dw);
+/* dW [Cin, Cout] = X^T dY over n rows each: the weight gradient of a 1x1x1 convolution, by the same kernel with
+ * the pairs (i, i) (workspace: tsmi_conv_wgrad_pairs_workspace_elems(n, 1, ...)). */
+int tsmi_conv_wgrad_pointwise(tsmi_stream_t s, const void *x, const void *dy, int64_t n, int cin, int cout,
+                              int dtype, float *workspace, int64_t workspace_elems, void *dw);
 
 /* Fetch-on-demand: one launch over 128-padded pair lists gathers X rows, multiplies
  * by W[k] and writes partial[qnbaddrs[k] + p, :] (fp32 for TSMI_F32, else the I/O
@@ -620,13 +627,42 @@ int tsmi_conv_implicit_gemm_packed(const int64_t *args);          /* 21 entries 
 int tsmi_conv_implicit_gemm_segments_packed(const int64_t *args); /* 20 entries */
 int tsmi_conv_implicit_gemm_grouped_packed(const int64_t *args);  /* 20 entries */
 
+/* One convolution y = act(sum_k X[map[:, k]] W[k] + bias + residual) as a struct, for callers that choose its form:
+ * over pair segments when in_rows is set (tsmi_conv_implicit_gemm_segments), over a grouped map when
+ * grouped is set (tsmi_conv_implicit_gemm_grouped), else over the map itself; fields of the other forms stay
+ * zero.  map NULL with kvol 1 is the identity (a 1x1x1 layer: n_map_rows = n_out).  ldy, y2, ldy2 place the
+ * result as above.  mirrored: offset k of the map takes W[kvol - 1 - k].  A submanifold map of distinct rows is its
+ * own transposed map with its offsets mirrored - map[i, k] = j where map[j, kvol - 1 - k] = i - so the input
+ * gradient of such a layer runs over the map, the segments and the grouping its forward has. */
+typedef struct {
+  tsmi_stream_t stream;
+  const void *x, *w_packed;
+  void *y, *y2;
+  int64_t ldy, ldy2;
+  const void *bias, *residual;
+  int32_t relu, dtype, kvol, cin, cout, mirrored;
+  int64_t n_out, n_map_rows;
+  const int32_t *map;
+  float *workspace;
+  int64_t workspace_elems;
+  int32_t *tile_counters;
+  int64_t n_tile_counters;
+  const int32_t *in_rows, *counts, *pos;
+  int64_t seg_rows;
+  void *products;
+  const int32_t *grouped, *row_of, *order64, *order128;
+  int64_t n_grouped;
+} tsmi_conv_call;
+int tsmi_conv(const tsmi_conv_call *call);
+
 /* A launch thread for the convolution calls of a forward (no counterpart in the reference, whose
  * calls are made one by one from the interpreter's thread).  Between _open and _close the three
  * packed convolution calls can be handed to one worker thread, which carries them out in the order
  * they were handed over while the caller prepares the next call: a call costs its caller ~0.5 us
  * instead of ~5.
  *   tsmi_launch_thread_submit(kind, args, n_words): kind 0 / 1 / 2 = tsmi_conv_implicit_gemm_packed
- *     / _segments_packed / _grouped_packed with the same argument block (copied).  Returns the
+ *     / _segments_packed / _grouped_packed with the same argument block (copied), kind 3 = tsmi_conv with
+ *     the struct as words (copied).  Returns the
  *     call's ticket (> 0), or -1 when no region is open (make the call yourself then).
  *   tsmi_launch_thread_completed(): address of an int64 that holds the ticket of the last call
  *     carried out.  The buffers of a submitted call must stay allocated until it has reached the
@@ -752,31 +788,35 @@ int tsmi_to_dense_backward(tsmi_stream_t s, const void *top_grad, const int32_t 
 
 /* ---- batch normalisation of feats [n, c] in training mode ------------------------------
  * Replaces what nn/modules/norm.py:13-17 reaches through torch.nn.BatchNorm1d on
- * SparseTensor.feats (forward with batch statistics, running-statistics update, backward).
- * x, y, dy, dx: [n, c] row-major of `dtype`, 16-byte aligned, c a multiple of 16 bytes' worth
+ * SparseTensor.feats (forward with batch statistics, running-statistics update, backward), with the
+ * activation and the shortcut that follow it in a network.
+ * x, y, dy, dx, residual, dz: [n, c] row-major of `dtype`, 16-byte aligned, c a multiple of 16 bytes' worth
  * of elements (8 for 16-bit types, 4 for fp32) and at most 256 such pieces.  weight, bias,
  * running_mean, running_var: [c] of `param_dtype`, each may be null (no affine term, no
- * running statistics).  partial: fp32 scratch of tsmi_bn_partial_elems(c) elements.  Sums run
- * in fp32 in a fixed order: results are identical from run to run.
+ * running statistics).  partial: fp32 scratch of tsmi_bn_partial_elems(c) elements; counters: 17 int32,
+ * zero before and after.  Sums run in fp32 in a fixed order: results are identical from run to run.
  *
- * forward:  stats[4c] (fp32) receives mean[c] and invstd[c] (biased variance,
- *           1/sqrt(var + eps)), which the backward takes, and 2c values of scratch;
- *           y = (x - mean) * invstd * weight + bias;
+ * forward:  stats[4c] (fp32) receives mean, 1/sqrt(biased var + eps), weight over that root, bias, which the
+ *           backward takes; y = act((x - mean) * invstd * weight + bias + residual), act the identity or
+ *           (relu) the clamp at zero;
  *           running_mean = (1 - momentum) * running_mean + momentum * mean,
- *           running_var likewise with the unbiased variance.
- * backward: sums[5c] (fp32) receives sum_rows dy (the bias gradient) in [0:c], sum_rows
- *           dy * xhat (the weight gradient) in [c:2c], xhat = (x - mean) * invstd, and 3c values
- *           of scratch; grads, when given, receives the same two gradients as [2c] of
- *           param_dtype;
- *           dx = weight * invstd * (dy - sums[0:c] / n - xhat * sums[c:2c] / n). */
+ *           running_var likewise with the unbiased variance; *batches += 1 where given.
+ * backward: g = dy where the activation passed (relu: where y > 0; y may be null for a layer without a
+ *           residual, whose sign is computed again from x), dz = g where given (the residual's
+ *           gradient); sums[5c] (fp32) receives sum_rows g (the bias gradient) in [0:c], sum_rows
+ *           g * xhat (the weight gradient) in [c:2c], xhat = (x - mean) * invstd, and 3c values
+ *           of scratch; grads, when given, receives the same two gradients as [2c] of param_dtype;
+ *           dx = weight * invstd * (g - sums[0:c] / n - xhat * sums[c:2c] / n).  stats needs its last 2c
+ *           values only for relu without y. */
 int64_t tsmi_bn_partial_elems(int c);
 int tsmi_bn_forward_train(tsmi_stream_t s, const void *x, int64_t n, int c, int dtype,
                           const void *weight, const void *bias, int param_dtype, void *running_mean,
-                          void *running_var, float momentum, float eps, float *partial, float *stats,
+                          void *running_var, int64_t *batches, float momentum, float eps,
+                          const void *residual, int relu, float *partial, int32_t *counters, float *stats,
                           void *y);
-int tsmi_bn_backward(tsmi_stream_t s, const void *dy, const void *x, int64_t n, int c, int dtype,
-                     const void *weight, int param_dtype, const float *mean, const float *invstd,
-                     float *partial, float *sums, void *grads, void *dx);
+int tsmi_bn_backward(tsmi_stream_t s, const void *dy, const void *x, const void *y, int64_t n, int c, int dtype,
+                     int relu, const void *weight, int param_dtype, float *stats, float *partial,
+                     int32_t *counters, float *sums, void *grads, void *dz, void *dx);
 
 #pragma GCC visibility pop
 #ifdef __cplusplus

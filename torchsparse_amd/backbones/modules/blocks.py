@@ -8,6 +8,7 @@ import numpy as np
 from torch import nn
 
 from ... import nn as spnn
+from ...nn.utils import stage
 from ...nn.utils.fuse import call_module
 from ...tensor import SparseTensor
 
@@ -28,6 +29,9 @@ class _Chain(nn.Sequential):
     place of folded norms and activations) instead of calling them."""
 
     def forward(self, x):
+        y = stage.run(self, x)
+        if y is not None:
+            return y
         for m in self._modules.values():
             if m.__class__ is not nn.Identity:
                 x = call_module(m, x)
@@ -67,6 +71,10 @@ class SparseResBlock(nn.Module):
     def forward(self, x: SparseTensor, also=None) -> SparseTensor:
         """``also``: a [N, out_channels] view the block's result is written into as well (the
         place a later concatenation wants it)."""
+        if also is None:
+            y = stage.run(self, x)
+            if y is not None:
+                return y
         if getattr(self, "_fused_tail", False):
             # after nn.utils.fuse_inference(): norms are folded into the convolutions and the
             # shortcut add + ReLU run in the epilogue of the block's last convolution

@@ -7,6 +7,7 @@ import torch
 from torch import nn
 
 from .. import nn as spnn
+from ..nn.utils import stage
 from ..operators import cat
 from ..tensor import SparseTensor
 from .modules import SparseConvBlock, SparseConvTransposeBlock, SparseResBlock
@@ -57,13 +58,13 @@ class SparseResUNet(nn.Module):
             plan = self.__dict__["_placed_plan"] = self._plan_placement()
         if plan and not self.training and x.feats.is_cuda:
             return self._forward_placed(x, plan)
-        skips = [self.stem(x)]
+        skips = [stage.call(self.stem, x)]
         for enc in self.encoders:
-            skips.append(enc(skips[-1]))
+            skips.append(stage.call(enc, skips[-1]))
         outputs = list(skips)
         y = skips[-1]
         for i, dec in enumerate(self.decoders):
-            y = dec["fuse"](cat([dec["upsample"](y), skips[3 - i]]))
+            y = stage.call(dec["fuse"], cat([dec["upsample"](y), skips[3 - i]]))
             outputs.append(y)
         return outputs
 
@@ -107,7 +108,14 @@ class SparseResUNet(nn.Module):
         from ..nn.utils.fuse import call_module
         skips, buffers = [], []
         y = x
-        for before, last, _, c_up, c_skip in plan:
+        stages = [self.stem] + list(self.encoders)[:3]
+        for (before, last, _, c_up, c_skip), whole in zip(plan, stages):
+            done = stage.run(whole, y, also=(c_up + c_skip, c_up))
+            if done is not None:
+                y, buf = done
+                skips.append(y)
+                buffers.append(buf)
+                continue
             for m in before:
                 y = call_module(m, y)
             buf = y.feats.new_empty(y.feats.shape[0], c_up + c_skip)
@@ -119,6 +127,11 @@ class SparseResUNet(nn.Module):
         for i, dec in enumerate(self.decoders):
             _, _, up, c_up, _ = plan[3 - i]
             buf = buffers[3 - i]
+            done = stage.run(dec["fuse"], y, modules=(dec["upsample"], dec["fuse"]), place=(buf, 0))
+            if done is not None:
+                y = done
+                outputs.append(y)
+                continue
             # (the result tensor of a call placed through a ColumnSlice is the whole buffer)
             y = call_module(dec["fuse"], call_module(up, y, out=ColumnSlice(buf, 0, c_up)))
             outputs.append(y)

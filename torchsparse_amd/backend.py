@@ -137,10 +137,11 @@ def _load():
         "tsmi_devoxelize_backward": [_vp, _vp, _vp, _vp, _vp, _i64, _i64, _i32, _i32, _vp],
         "tsmi_to_dense_forward": [_vp, _vp, _vp, _i64, _i32, _I4, _i32, _vp],
         "tsmi_to_dense_backward": [_vp, _vp, _vp, _i64, _i32, _I4, _i32, _vp],
-        "tsmi_bn_forward_train": [_vp, _vp, _i64, _i32, _i32, _vp, _vp, _i32, _vp, _vp, _f32, _f32, _vp, _vp,
-                                  _vp],
+        "tsmi_bn_forward_train": [_vp, _vp, _i64, _i32, _i32, _vp, _vp, _i32, _vp, _vp, _vp, _f32, _f32, _vp,
+                                  _i32, _vp, _vp, _vp, _vp],
         "tsmi_bn_partial_elems": [_i32],
-        "tsmi_bn_backward": [_vp, _vp, _vp, _i64, _i32, _i32, _vp, _i32, _vp, _vp, _vp, _vp, _vp, _vp],
+        "tsmi_bn_backward": [_vp, _vp, _vp, _vp, _i64, _i32, _i32, _i32, _vp, _i32, _vp, _vp, _vp, _vp, _vp, _vp,
+                             _vp],
         "tsmi_gs_gather": [_vp, _vp, _vp, _i64, _i32, _i32, _i32, _vp],
         "tsmi_gs_gemm": [_vp, _vp, _vp, _vp, _vp, _i64, _i64, _i32, _i32, _i32, _i32, _vp],
         "tsmi_gs_scatter": [_vp, _vp, _vp, _vp, _i64, _i32, _i32, _i32, _i32, _vp, _vp, _i32, _vp],
@@ -1314,6 +1315,8 @@ def release_scratch() -> None:
         _stream_states.clear()
     with _scratch_lock:
         _SCRATCH.clear()
+    if _native_module is not None:
+        _native_module.release_scratch()
 
 
 def _grid_layout(words0: int):
@@ -1935,12 +1938,26 @@ def _hand_over(kind: int, block: bytes, words: int, keep) -> bool:
     ticket = _C.tsmi_launch_thread_submit(kind, block, words)
     if ticket < 0:
         return False
+    _keep_until(ticket, keep)
+    return True
+
+
+def _keep_until(ticket: int, keep) -> None:
     calls = _region_calls
     done = _completed.value
     while calls and calls[0][0] <= done:
         calls.popleft()
     calls.append((ticket, keep))
-    return True
+
+
+def pending_calls():
+    """For a native stage inside a region: collects what its calls, which go to the launch thread, need kept."""
+    return native().Pending() if _region_depth else None
+
+
+def keep_pending(pending) -> None:
+    if pending.ticket:
+        _keep_until(pending.ticket, pending)
 
 
 _PACK20 = struct.Struct("20q").pack
@@ -2493,6 +2510,58 @@ def _implicit_gemm(x, wp, kvol, cin, cout, out_in_map, num_out_feats, bias=None,
     return y
 
 
+# ---- the native host path (csrc/native: stages of convolutions, nn/utils/stage.py)
+
+_native_module = None
+
+
+def native():
+    """The native module, loaded on first use (it links against torch's GPU libraries)."""
+    global _native_module
+    if _native_module is None:
+        from . import _native
+        _native_module = _native
+    return _native_module
+
+
+@functools.lru_cache(maxsize=64)
+def native_identity(n: int):
+    """The map of a 1x1x1 layer over n rows (no table: the kernels know it)."""
+    return native().KernelMap(1, n, n, True, None, None)
+
+
+def native_segments(handle, x, channels, kmap, force) -> bool:
+    """Whether layers of a submanifold or strided map run over its pair segments, given the channels
+    of one that could (kernel volume, inputs, outputs); attaches the segments to the map's handle."""
+    if handle.has_segments:
+        return True
+    omap, n = kmap["out_in_map"], kmap["sizes"][1]
+    if n >= 65536 or not _segments_pay(x, *channels, n, omap, force):
+        return False
+    seg = pair_segments(omap, n)
+    handle.set_segments(seg.buffer, seg.in_rows_ptr, seg.counts_ptr, seg.pos_ptr, seg.seg_rows)
+    return True
+
+
+def native_grouped(handle, kmap, uses: int) -> None:
+    """Attaches the grouped copy of a 3x3x3 map that has served enough layers (``uses`` more now)."""
+    n = kmap["sizes"][1]
+    omap = kmap["out_in_map"]
+    if not igemm_group_rows or handle.has_grouped or n < group_min_rows or omap.shape[1] != 27:
+        return
+    if igemm_group_rows != "always":
+        key = id(omap)
+        hit = _group_uses.get(key)
+        if (hit is None or hit[0]() is not omap or hit[1] != omap._version or hit[2] != omap.data_ptr()):
+            hit = [weakref.ref(omap), omap._version, omap.data_ptr(), 0]
+            _remember(_group_uses, key, hit, 256)
+        hit[3] += uses
+        if hit[3] < group_after_uses or torch.cuda.is_current_stream_capturing():
+            return
+    g = grouped_map(omap, n)
+    handle.set_grouped(g.buffer, list(g.ptrs), g.padded)
+
+
 _IDENTITY_MAPS = {}
 
 
@@ -2995,12 +3064,14 @@ def bn_forward_train(x, weight, bias, running_mean, running_var, momentum: float
     n, c = x.shape
     given = [p for p in (weight, bias, running_mean, running_var) if p is not None]
     pcode = _dtype_code(given[0]) if given else F32
+    stream = _stream()
     work = torch.empty(_C.tsmi_bn_partial_elems(c), dtype=torch.float32, device=x.device)
     stats = torch.empty(4 * c, dtype=torch.float32, device=x.device)
     y = torch.empty_like(x)
-    _check(_C.tsmi_bn_forward_train(_stream(), _ptr(x), n, c, _dtype_code(x), _ptr(weight), _ptr(bias), pcode,
-                                    _ptr(running_mean), _ptr(running_var), float(momentum), float(eps),
-                                    _ptr(work), _ptr(stats), _ptr(y)))
+    _check(_C.tsmi_bn_forward_train(stream, _ptr(x), n, c, _dtype_code(x), _ptr(weight), _ptr(bias), pcode,
+                                    _ptr(running_mean), _ptr(running_var), None, float(momentum), float(eps),
+                                    None, 0, _ptr(work), _tile_counters(x.device, stream).data_ptr(), _ptr(stats),
+                                    _ptr(y)))
     return y, stats[:c], stats[c:2 * c]
 
 
@@ -3008,13 +3079,17 @@ def bn_backward(dy, x, weight, mean, invstd):
     """(dx, sum_rows dy * xhat, sum_rows dy): the input, weight and bias gradients (the last two in
     the weight's type; fp32 without a weight)."""
     n, c = x.shape
+    stream = _stream()
+    if invstd.data_ptr() != mean.data_ptr() + 4 * c:  # (the two halves of what bn_forward_train returned)
+        mean = torch.cat((mean.float(), invstd.float()))
     work = torch.empty(_C.tsmi_bn_partial_elems(c), dtype=torch.float32, device=x.device)
     sums = torch.empty(5 * c, dtype=torch.float32, device=x.device)
     dx = torch.empty_like(x)
     pcode = _dtype_code(weight) if weight is not None else F32
     grads = torch.empty(2 * c, dtype=weight.dtype, device=x.device) if weight is not None else None
-    _check(_C.tsmi_bn_backward(_stream(), _ptr(dy), _ptr(x), n, c, _dtype_code(x), _ptr(weight), pcode,
-                               _ptr(mean), _ptr(invstd), _ptr(work), _ptr(sums), _ptr(grads), _ptr(dx)))
+    _check(_C.tsmi_bn_backward(stream, _ptr(dy), _ptr(x), None, n, c, _dtype_code(x), 0, _ptr(weight), pcode,
+                               _ptr(mean), _ptr(work), _tile_counters(x.device, stream).data_ptr(), _ptr(sums),
+                               _ptr(grads), None, _ptr(dx)))
     if grads is not None:
         return dx, grads[c:], grads[:c]
     return dx, sums[c:2 * c], sums[:c]

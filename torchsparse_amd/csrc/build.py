@@ -2,6 +2,8 @@
 
   python torchsparse_amd/csrc/build.py [-v]
 
+and the native host path over torch's C++ API into torchsparse_amd/_native.so.
+
 hipcc cross-compiles without a GPU; the shared object stays in-tree.
 """
 import os
@@ -64,9 +66,39 @@ def _compile(src, verbose):
     return obj
 
 
+NATIVE = os.path.join(PKG, "_native.so")
+
+
+def _compile_native(verbose):
+    """The object of csrc/native/native.cpp: host code only, against torch's headers."""
+    import sysconfig
+
+    from torch.utils import cpp_extension
+    obj = os.path.join(OBJ_DIR, "native.o")
+    include = [f"-I{p}" for p in cpp_extension.include_paths("cuda") + [sysconfig.get_paths()["include"]]]
+    cmd = ["g++", "-O2", "-std=c++17", "-fPIC", "-fvisibility=hidden", "-D__HIP_PLATFORM_AMD__", "-DUSE_ROCM",
+           "-DTORCH_API_INCLUDE_EXTENSION_H", "-DTORCH_EXTENSION_NAME=_native", "-Wno-attributes"] + include
+    cmd += ["-c", os.path.join(HERE, "native", "native.cpp"), "-o", obj]
+    if verbose:
+        print(" ".join(cmd), flush=True)
+    r = subprocess.run(cmd, capture_output=True, text=True)
+    if r.returncode != 0:
+        raise RuntimeError(f"g++ failed on native.cpp:\n{r.stderr}")
+    return obj
+
+
+def _link_native(obj):
+    import torch
+    lib = os.path.join(os.path.dirname(torch.__file__), "lib")
+    subprocess.check_call(["g++", "-shared", "-o", NATIVE, obj, f"-L{PKG}", "-l:libtsmi.so", f"-L{lib}", "-lc10",
+                           "-ltorch_cpu", "-ltorch", "-ltorch_python", "-lc10_hip", "-ltorch_hip",
+                           "-Wl,-rpath,$ORIGIN"])
+
+
 def build(verbose: bool = False, jobs: int = 8) -> str:
     os.makedirs(OBJ_DIR, exist_ok=True)
     with ThreadPoolExecutor(max_workers=jobs) as ex:
+        native = None if SANITIZE else ex.submit(_compile_native, verbose)
         objs = list(ex.map(lambda s: _compile(s, verbose), SOURCES))
     cmd = [HIPCC, "--offload-arch=gfx950", "-shared", "-fPIC", "-o", OUT] + objs
     if SANITIZE:
@@ -74,6 +106,8 @@ def build(verbose: bool = False, jobs: int = 8) -> str:
     if verbose:
         print(" ".join(cmd), flush=True)
     subprocess.check_call(cmd)
+    if native is not None:
+        _link_native(native.result())
     return OUT
 
 

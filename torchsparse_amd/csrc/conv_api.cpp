@@ -2,6 +2,8 @@
 // the element type.  The kernels live in conv_igemm.inc.
 #include "conv_ops.h"
 
+#include <vector>
+
 using namespace tsmi;
 
 namespace {
@@ -37,7 +39,21 @@ extern "C" int tsmi_pack_weights(tsmi_stream_t s, const void *w, void *w_packed,
   const ConvOps *ops = ops_for(dtype);
   if (int e = check_shapes("pack_weights", ops, kvol, cin, cout)) return e;
   TSMI_REQUIRE(w && w_packed, "pack_weights: null pointer");
-  return ops->pack((hipStream_t)s, w, w_packed, kvol, cin, cout);
+  const PackJob job{w, w_packed, kvol, cin, cout};
+  return ops->pack((hipStream_t)s, &job, 1);
+}
+
+extern "C" int tsmi_pack_weights_many(tsmi_stream_t s, const void *const *w, void *const *w_packed,
+                                      const int32_t *shapes, int n, int dtype) {
+  const ConvOps *ops = ops_for(dtype);
+  TSMI_REQUIRE(n >= 0 && (n == 0 || (w && w_packed && shapes)), "pack_weights_many: bad arguments");
+  std::vector<PackJob> jobs(n);
+  for (int i = 0; i < n; ++i) {
+    if (int e = check_shapes("pack_weights_many", ops, shapes[3 * i], shapes[3 * i + 1], shapes[3 * i + 2])) return e;
+    TSMI_REQUIRE(w[i] && w_packed[i], "pack_weights_many: null pointer");
+    jobs[i] = PackJob{w[i], w_packed[i], shapes[3 * i], shapes[3 * i + 1], shapes[3 * i + 2]};
+  }
+  return n == 0 ? TSMI_OK : ops->pack((hipStream_t)s, jobs.data(), n);
 }
 
 extern "C" int64_t tsmi_conv_workspace_elems(int64_t n_tile_rows, int64_t n_out, int kvol,
@@ -71,7 +87,7 @@ static int implicit_gemm(tsmi_stream_t s, const void *x, const void *w_packed, c
   TSMI_REQUIRE(n_out >= 0 && n_map_rows >= n_out, "conv_implicit_gemm: map has %lld rows, need %lld",
                (long long)n_map_rows, (long long)n_out);
   if (n_out == 0) return TSMI_OK;
-  TSMI_REQUIRE(x && w_packed && map && y, "conv_implicit_gemm: null pointer");
+  TSMI_REQUIRE(x && w_packed && (map || (kvol == 1 && place)) && y, "conv_implicit_gemm: null pointer");
   TSMI_REQUIRE(aligned16(x) && aligned16(w_packed) && aligned16(y),
                "conv_implicit_gemm: x, w_packed and y must be 16-byte aligned");
   return ops->igemm((hipStream_t)s, x, w_packed, map, n_map_rows, n_out, n_out, kvol, cin, cout,
@@ -189,8 +205,20 @@ extern "C" int tsmi_conv_wgrad_pairs(tsmi_stream_t s, const void *x, const void 
   TSMI_REQUIRE(pair_cap == 0 || (x && dy && pairs), "conv_wgrad_pairs: null pointer");
   TSMI_REQUIRE(aligned16(x) && aligned16(dy) && ((uintptr_t)pairs & 7) == 0,
                "conv_wgrad_pairs: x and dy must be 16-byte aligned, pairs 8-byte aligned");
-  return ops->wgrad_pairs((hipStream_t)s, x, dy, pairs, seg_steps, pair_cap, x_col, kvol, cin, cout,
+  return ops->wgrad_pairs((hipStream_t)s, x, dy, pairs, seg_steps, pair_cap, x_col, kvol, cin, cout, 0,
                           workspace, workspace_elems, dw);
+}
+
+extern "C" int tsmi_conv_wgrad_pointwise(tsmi_stream_t s, const void *x, const void *dy, int64_t n, int cin,
+                                         int cout, int dtype, float *workspace, int64_t workspace_elems,
+                                         void *dw) {
+  const ConvOps *ops = ops_for(dtype);
+  if (int e = check_shapes("conv_wgrad_pointwise", ops, 1, cin, cout)) return e;
+  TSMI_REQUIRE(n > 0 && n < (int64_t(1) << 31) - kWgradPairStep, "conv_wgrad_pointwise: %lld rows", (long long)n);
+  TSMI_REQUIRE(x && dy && dw && workspace && aligned16(x) && aligned16(dy),
+               "conv_wgrad_pointwise: null or misaligned pointer");
+  return ops->wgrad_pairs((hipStream_t)s, x, dy, nullptr, nullptr, n, 0, 1, cin, cout, n, workspace,
+                          workspace_elems, dw);
 }
 
 extern "C" int tsmi_conv_fetch_on_demand(tsmi_stream_t s, const void *x, const void *w_packed,
@@ -244,7 +272,7 @@ static int implicit_gemm_segments(tsmi_stream_t s, const void *x, const void *w_
   TSMI_REQUIRE(aligned16(x) && aligned16(w_packed) && aligned16(products) && aligned16(y),
                "conv_implicit_gemm_segments: x, w_packed, products and y must be 16-byte aligned");
   if (int e = ops->segments((hipStream_t)s, x, w_packed, in_rows, counts, seg_rows, kvol, cin, cout,
-                            products))
+                            place ? place->mirrored : 0, products))
     return e;
   return ops->segment_sum((hipStream_t)s, products, pos, n_out, kvol, seg_rows, cout, bias, residual,
                           relu, y, place);
@@ -310,6 +338,7 @@ static const OutPlace *place_of(const int64_t *w, OutPlace *place) {
   place->ldy = w[0];
   place->y2 = (void *)as_ptr(w[1]);
   place->ldy2 = w[2];
+  place->mirrored = 0;
   return place;
 }
 
@@ -340,4 +369,21 @@ extern "C" int tsmi_conv_implicit_gemm_segments_packed(const int64_t *a) {
                                 (const int32_t *)as_ptr(a[5]), a[6], a[7], (int)a[8], (int)a[9],
                                 (int)a[10], (int)a[11], as_ptr(a[12]), as_ptr(a[13]), (int)a[14],
                                 (void *)as_ptr(a[15]), (void *)as_ptr(a[16]), place_of(a + 17, &place));
+}
+
+// One convolution in whichever form the caller has products of the map for.
+extern "C" int tsmi_conv(const tsmi_conv_call *c) {
+  TSMI_REQUIRE(c, "conv: null call");
+  OutPlace place{c->ldy, c->y2, c->ldy2, c->mirrored};
+  if (c->in_rows)
+    return implicit_gemm_segments(c->stream, c->x, c->w_packed, c->in_rows, c->counts, c->pos, c->seg_rows, c->n_out,
+                                  c->kvol, c->cin, c->cout, c->dtype, c->bias, c->residual, c->relu, c->products,
+                                  c->y, &place);
+  if (c->grouped)
+    return implicit_gemm_grouped(c->stream, c->x, c->w_packed, c->grouped, c->row_of, c->order64, c->order128,
+                                 c->n_grouped, c->n_out, c->kvol, c->cin, c->cout, c->dtype, c->bias, c->residual,
+                                 c->relu, c->y, &place);
+  return implicit_gemm(c->stream, c->x, c->w_packed, c->map, c->n_map_rows, c->n_out, c->kvol, c->cin, c->cout,
+                       c->dtype, c->bias, c->residual, c->relu, c->workspace, c->workspace_elems, c->tile_counters,
+                       c->n_tile_counters, c->y, &place);
 }

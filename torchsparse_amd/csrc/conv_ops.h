@@ -18,11 +18,19 @@ struct OutPlace {
   int64_t ldy;
   void *y2;
   int64_t ldy2;
+  int mirrored;  // not 0: offset k of the map takes the weights of offset kvol - 1 - k
+};
+
+// One weight tensor [kvol, cin, cout] on its way to the packed layout [kvol, cout_pad, cin_pad].
+struct PackJob {
+  const void *w;
+  void *wp;
+  int kvol, cin, cout;
 };
 
 struct ConvOps {
   int step;  // reduction elements per MFMA step (Cin is padded to a multiple)
-  int (*pack)(hipStream_t s, const void *w, void *wp, int kvol, int cin, int cout);
+  int (*pack)(hipStream_t s, const PackJob *jobs, int n);
   // floats of scratch igemm wants for this problem (0 = none)
   int64_t (*workspace)(int64_t n_tile_rows, int64_t n_out, int kvol, int split, int cin, int cout,
                        int sorted);
@@ -50,16 +58,17 @@ struct ConvOps {
   int64_t (*wgrad_workspace)(int64_t n_in, int kvol, int cin, int cout);
   int (*wgrad)(hipStream_t s, const void *x, const void *dy, const int32_t *map_bwd, int64_t n_in,
                int kvol, int cin, int cout, float *partial, int64_t partial_elems, void *dw);
-  // the same sums over padded pair lists (tsmi_wgrad_pairs_build); pairs[:, x_col] indexes x
+  // the same sums over padded pair lists (tsmi_wgrad_pairs_build); pairs[:, x_col] indexes x.  identity > 0:
+  // no lists but the pairs (i, i), i < identity, of one offset
   int64_t (*wgrad_pairs_workspace)(int64_t pair_cap, int kvol, int cin, int cout);
   int (*wgrad_pairs)(hipStream_t s, const void *x, const void *dy, const int32_t *pairs,
                      const int32_t *seg_steps, int64_t pair_cap, int x_col, int kvol, int cin,
-                     int cout, float *partial, int64_t partial_elems, void *dw);
+                     int cout, int64_t identity, float *partial, int64_t partial_elems, void *dw);
   // 1 when `segments` has a variant for the shape
   int (*segments_supported)(int kvol, int cin, int cout);
   // products[k * seg_rows + j, :] = X[in_rows[k * seg_rows + j], :] W[k] for j < counts[k]
   int (*segments)(hipStream_t s, const void *x, const void *wp, const int32_t *in_rows,
-                  const int32_t *counts, int64_t seg_rows, int kvol, int cin, int cout,
+                  const int32_t *counts, int64_t seg_rows, int kvol, int cin, int cout, int mirrored,
                   void *products);
   // y[o, :] = sum over k of products[k * seg_rows + pos[k * n_out + o], :] where pos >= 0
   int (*segment_sum)(hipStream_t s, const void *products, const int32_t *pos, int64_t n_out, int kvol,

@@ -2,7 +2,7 @@
 //
 // A forward of a network makes ~60 convolution calls; each costs the calling thread ~5 us inside
 // the library (argument checks, the plan, hipLaunchKernel) on top of the ~5 us its binding spends
-// preparing it.  Between tsmi_launch_thread_open and _close the three packed convolution calls
+// preparing it.  Between tsmi_launch_thread_open and _close the convolution calls
 // can be handed to ONE worker thread instead (tsmi_launch_thread_submit): the worker carries them
 // out in the order they were handed over, while the caller prepares the next one.  Launches
 // reach each stream in submission order; everything else the caller does on those streams itself
@@ -23,10 +23,12 @@
 namespace {
 
 constexpr int kRing = 256;
-constexpr int kWords = 21;
+constexpr int kWords = sizeof(tsmi_conv_call) / sizeof(int64_t);
+static_assert(sizeof(tsmi_conv_call) % sizeof(int64_t) == 0 && kWords >= 21, "a job holds any of the argument blocks");
 
 struct Job {
-  int kind;    // 0: tsmi_conv_implicit_gemm_packed, 1: ..._segments_packed, 2: ..._grouped_packed
+  int kind;    // 0: tsmi_conv_implicit_gemm_packed, 1: ..._segments_packed, 2: ..._grouped_packed,
+               // 3: tsmi_conv
   int device;  // the device that was current when the call was handed over
   int64_t a[kWords];
 };
@@ -58,7 +60,8 @@ void run_job(const Job &j, int *current_device) {
   switch (j.kind) {
     case 0: status = tsmi_conv_implicit_gemm_packed(j.a); break;
     case 1: status = tsmi_conv_implicit_gemm_segments_packed(j.a); break;
-    default: status = tsmi_conv_implicit_gemm_grouped_packed(j.a); break;
+    case 2: status = tsmi_conv_implicit_gemm_grouped_packed(j.a); break;
+    default: status = tsmi_conv(reinterpret_cast<const tsmi_conv_call *>(j.a)); break;
   }
   if (status != TSMI_OK && !g_error.load()) {
     strncpy(g_message, tsmi_last_error(), sizeof(g_message) - 1);  // (the worker's own last error)
@@ -110,7 +113,7 @@ extern "C" int tsmi_launch_thread_open(void) {
 }
 
 extern "C" int64_t tsmi_launch_thread_submit(int kind, const int64_t *args, int n_words) {
-  if (kind < 0 || kind > 2 || !args || n_words < 1 || n_words > kWords || g_open.load() <= 0) return -1;
+  if (kind < 0 || kind > 3 || !args || n_words < 1 || n_words > kWords || g_open.load() <= 0) return -1;
   int device = 0;
   if (hipGetDevice(&device) != hipSuccess) return -1;
   std::lock_guard<std::mutex> lock(g_submit_mutex);

@@ -10,7 +10,7 @@ from .func import (FetchOnDemandConvolutionFuntion, GatherScatterConvolutionFunt
                    ImplicitGEMMConvolutionFuntion)
 from .kmap import build_kernel_map, transpose_kernel_map
 
-__all__ = ["conv3d", "conv3d_cached"]
+__all__ = ["conv3d", "conv3d_cached", "kernel_map"]
 
 _DATAFLOWS = {
     _cfg.Dataflow.ImplicitGEMM: ImplicitGEMMConvolutionFuntion,
@@ -99,19 +99,7 @@ def conv3d(input: SparseTensor, weight: torch.Tensor,
         out_stride = (ist[0] * stride[0], ist[1] * stride[1], ist[2] * stride[2])
         kmap = caches.kmaps.get(key)
         if kmap is None:
-            in_hashmap = caches.hashmaps.get(input.stride)
-            keys, vals = in_hashmap if in_hashmap is not None else (None, None)
-            kmap = build_kernel_map(
-                coords, feats.shape[0], kernel_size, stride, padding, keys, vals,
-                input.spatial_range, config["kmap_mode"], dataflow,
-                downsample_mode=config["downsample_mode"], training=training,
-                ifsort=config["ifsort"], split_mask_num=config["split_mask_num"],
-                split_mask_num_bwd=config["split_mask_num_bwd"])
-            caches.kmaps[key] = kmap
-            # tables exist only where a map was built through one (unsorted coordinates, "hashmap" mode)
-            for level, table in ((input.stride, kmap["in_hashmap"]), (out_stride, kmap["out_hashmap"])):
-                if table is not None and caches.hashmaps.get(level) is None:
-                    caches.hashmaps[level] = table
+            kmap = kernel_map(caches, key, coords, feats.shape[0], padding, input.spatial_range, config, training)
         if (weight.dim() == 3 and feats.shape[1] == weight.shape[1]
                 and _direct_ok(feats, weight, bias, residual, config)):
             # (what conv_fn.apply comes down to for an inference call in the unsorted implicit GEMM)
@@ -174,6 +162,26 @@ def conv3d(input: SparseTensor, weight: torch.Tensor,
     if output.stride not in caches.cmaps:
         caches.cmaps[output.stride] = (output.coords, output.spatial_range)
     return output
+
+
+def kernel_map(caches, key, coords: torch.Tensor, n_in: int, padding, spatial_range, config: Dict,
+               training: bool) -> Dict:
+    """The kernel map of the non-transposed geometry ``key`` = (input stride, kernel size, stride,
+    dilation), built over the input level's ``coords`` and put into the tensor's caches."""
+    in_stride, kernel_size, stride, _ = key
+    keys, vals = caches.hashmaps.get(in_stride) or (None, None)
+    kmap = build_kernel_map(
+        coords, n_in, kernel_size, stride, padding, keys, vals, spatial_range, config["kmap_mode"],
+        config["dataflow"], downsample_mode=config["downsample_mode"], training=training,
+        ifsort=config["ifsort"], split_mask_num=config["split_mask_num"],
+        split_mask_num_bwd=config["split_mask_num_bwd"])
+    caches.kmaps[key] = kmap
+    # tables exist only where a map was built through one (unsorted coordinates, "hashmap" mode)
+    out_stride = tuple(in_stride[a] * stride[a] for a in range(3))
+    for level, table in ((in_stride, kmap["in_hashmap"]), (out_stride, kmap["out_hashmap"])):
+        if table is not None and caches.hashmaps.get(level) is None:
+            caches.hashmaps[level] = table
+    return kmap
 
 
 def _direct_ok(feats, kernel, bias, residual, config) -> bool:

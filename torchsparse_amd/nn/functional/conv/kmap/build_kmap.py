@@ -38,6 +38,29 @@ def _empty_kmap(hashmap_keys, hashmap_vals, spatial_range) -> Dict:
     return kmap
 
 
+class _TrainingMap(dict):
+    """A kernel map whose backward products (the ``*_bwd`` keys) are built when one of them is first
+    looked at: a submanifold map over distinct rows is its own transposed map with its offsets
+    mirrored, and a strided one often has been transposed already, so most layers never need them."""
+    _NAMES = frozenset(("out_in_map_bwd", "reorder_out_in_map_bwd", "reduced_sorted_mask_bwd_wgrad",
+                        "reduced_sorted_mask_bwd_dgrad", "reorder_loc_bwd"))
+    products = None  # (ifsort, split_mask_num_bwd) while they are not built
+
+    def _settle(self):
+        todo, self.products = self.products, None
+        _backward_products(self, *todo)
+
+    def __getitem__(self, key):
+        if self.products is not None and key in self._NAMES:
+            self._settle()
+        return dict.__getitem__(self, key)
+
+    def get(self, key, default=None):
+        if self.products is not None and key in self._NAMES:
+            self._settle()
+        return dict.get(self, key, default)
+
+
 def _strided_range(spatial_range, kernel_size, stride, padding):
     """(B, X', Y', Z') with X' = (X + 2p - (k-1) - 1)//s + 1 — build_kmap.py:65-72."""
     if spatial_range is None:
@@ -236,6 +259,8 @@ def build_kernel_map(_coords: torch.Tensor, input_node_num: int,
         return None if table is None else (table.keys, table.vals)
 
     kmap["out_in_map"] = out_in_map
+    # every row of the map stands for a cell of its own (rows found by search ascend strictly)
+    kmap["distinct"] = by_search
     kmap["subm"] = subm  # stride 1: outputs are the inputs, the centre offset is the identity
     kmap["coords"] = out_coords if not subm else _coords
     kmap["sizes"] = (input_node_num, out_coords.shape[0])
@@ -249,7 +274,8 @@ def build_kernel_map(_coords: torch.Tensor, input_node_num: int,
         if ifsort:
             _sort_products(kmap, out_in_map, kmap["sizes"][1], split_mask_num)
         if training:
-            _backward_products(kmap, ifsort, split_mask_num_bwd)
+            kmap = _TrainingMap(kmap)
+            kmap.products = (ifsort, split_mask_num_bwd)
     else:
         _pair_products(kmap, dataflow)
     return kmap

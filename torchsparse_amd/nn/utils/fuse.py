@@ -71,6 +71,10 @@ class FoldedSequential(nn.Sequential):
     forward of a 42-layer U-Net."""
 
     def forward(self, x):
+        from . import stage
+        y = stage.run(self, x)
+        if y is not None:
+            return y
         for m in self._modules.values():
             if m.__class__ is not nn.Identity:
                 x = call_module(m, x)
