@@ -793,8 +793,8 @@ int tsmi_to_dense_backward(tsmi_stream_t s, const void *top_grad, const int32_t 
  * x, y, dy, dx, residual, dz: [n, c] row-major of `dtype`, 16-byte aligned, c a multiple of 16 bytes' worth
  * of elements (8 for 16-bit types, 4 for fp32) and at most 256 such pieces.  weight, bias,
  * running_mean, running_var: [c] of `param_dtype`, each may be null (no affine term, no
- * running statistics).  partial: fp32 scratch of tsmi_bn_partial_elems(c) elements; counters: 17 int32,
- * zero before and after.  Sums run in fp32 in a fixed order: results are identical from run to run.
+ * running statistics).  partial: fp32 scratch of tsmi_bn_partial_elems(c) elements, 16-byte aligned.
+ * Sums run in fp32 in a fixed order: results are identical from run to run.
  *
  * forward:  stats[4c] (fp32) receives mean, 1/sqrt(biased var + eps), weight over that root, bias, which the
  *           backward takes; y = act((x - mean) * invstd * weight + bias + residual), act the identity or
@@ -803,20 +803,18 @@ int tsmi_to_dense_backward(tsmi_stream_t s, const void *top_grad, const int32_t 
  *           running_var likewise with the unbiased variance; *batches += 1 where given.
  * backward: g = dy where the activation passed (relu: where y > 0; y may be null for a layer without a
  *           residual, whose sign is computed again from x), dz = g where given (the residual's
- *           gradient); sums[5c] (fp32) receives sum_rows g (the bias gradient) in [0:c], sum_rows
- *           g * xhat (the weight gradient) in [c:2c], xhat = (x - mean) * invstd, and 3c values
- *           of scratch; grads, when given, receives the same two gradients as [2c] of param_dtype;
+ *           gradient); sums[2c] (fp32) receives sum_rows g (the bias gradient) and sum_rows
+ *           g * xhat (the weight gradient), xhat = (x - mean) * invstd; grads, when given, receives the same two gradients as [2c] of param_dtype;
  *           dx = weight * invstd * (g - sums[0:c] / n - xhat * sums[c:2c] / n).  stats needs its last 2c
  *           values only for relu without y. */
 int64_t tsmi_bn_partial_elems(int c);
 int tsmi_bn_forward_train(tsmi_stream_t s, const void *x, int64_t n, int c, int dtype,
                           const void *weight, const void *bias, int param_dtype, void *running_mean,
                           void *running_var, int64_t *batches, float momentum, float eps,
-                          const void *residual, int relu, float *partial, int32_t *counters, float *stats,
-                          void *y);
+                          const void *residual, int relu, float *partial, float *stats, void *y);
 int tsmi_bn_backward(tsmi_stream_t s, const void *dy, const void *x, const void *y, int64_t n, int c, int dtype,
                      int relu, const void *weight, int param_dtype, float *stats, float *partial,
-                     int32_t *counters, float *sums, void *grads, void *dz, void *dx);
+                     float *sums, void *grads, void *dz, void *dx);
 
 #pragma GCC visibility pop
 #ifdef __cplusplus

@@ -138,9 +138,9 @@ def _load():
         "tsmi_to_dense_forward": [_vp, _vp, _vp, _i64, _i32, _I4, _i32, _vp],
         "tsmi_to_dense_backward": [_vp, _vp, _vp, _i64, _i32, _I4, _i32, _vp],
         "tsmi_bn_forward_train": [_vp, _vp, _i64, _i32, _i32, _vp, _vp, _i32, _vp, _vp, _vp, _f32, _f32, _vp,
-                                  _i32, _vp, _vp, _vp, _vp],
+                                  _i32, _vp, _vp, _vp],
         "tsmi_bn_partial_elems": [_i32],
-        "tsmi_bn_backward": [_vp, _vp, _vp, _vp, _i64, _i32, _i32, _i32, _vp, _i32, _vp, _vp, _vp, _vp, _vp, _vp,
+        "tsmi_bn_backward": [_vp, _vp, _vp, _vp, _i64, _i32, _i32, _i32, _vp, _i32, _vp, _vp, _vp, _vp, _vp,
                              _vp],
         "tsmi_gs_gather": [_vp, _vp, _vp, _i64, _i32, _i32, _i32, _vp],
         "tsmi_gs_gemm": [_vp, _vp, _vp, _vp, _vp, _i64, _i64, _i32, _i32, _i32, _i32, _vp],
@@ -3070,8 +3070,7 @@ def bn_forward_train(x, weight, bias, running_mean, running_var, momentum: float
     y = torch.empty_like(x)
     _check(_C.tsmi_bn_forward_train(stream, _ptr(x), n, c, _dtype_code(x), _ptr(weight), _ptr(bias), pcode,
                                     _ptr(running_mean), _ptr(running_var), None, float(momentum), float(eps),
-                                    None, 0, _ptr(work), _tile_counters(x.device, stream).data_ptr(), _ptr(stats),
-                                    _ptr(y)))
+                                    None, 0, _ptr(work), _ptr(stats), _ptr(y)))
     return y, stats[:c], stats[c:2 * c]
 
 
@@ -3083,12 +3082,12 @@ def bn_backward(dy, x, weight, mean, invstd):
     if invstd.data_ptr() != mean.data_ptr() + 4 * c:  # (the two halves of what bn_forward_train returned)
         mean = torch.cat((mean.float(), invstd.float()))
     work = torch.empty(_C.tsmi_bn_partial_elems(c), dtype=torch.float32, device=x.device)
-    sums = torch.empty(5 * c, dtype=torch.float32, device=x.device)
+    sums = torch.empty(2 * c, dtype=torch.float32, device=x.device)
     dx = torch.empty_like(x)
     pcode = _dtype_code(weight) if weight is not None else F32
     grads = torch.empty(2 * c, dtype=weight.dtype, device=x.device) if weight is not None else None
     _check(_C.tsmi_bn_backward(stream, _ptr(dy), _ptr(x), None, n, c, _dtype_code(x), 0, _ptr(weight), pcode,
-                               _ptr(mean), _ptr(work), _tile_counters(x.device, stream).data_ptr(), _ptr(sums),
+                               _ptr(mean), _ptr(work), _ptr(sums),
                                _ptr(grads), None, _ptr(dx)))
     if grads is not None:
         return dx, grads[c:], grads[:c]

@@ -469,21 +469,17 @@ torch::autograd::variable_list StageNode::apply(torch::autograd::variable_list &
       const Tensor &c = conv_out[i];
       const int ch = op.cout;
       const Tensor &w = op.norm.gamma >= 0 ? weights[op.norm.gamma] : c;
-      const Tensor work = floats(tsmi_bn_partial_elems(ch) + 5 * ch, x);
+      const Tensor work = floats(tsmi_bn_partial_elems(ch) + 2 * ch, x);
       float *partial = work.data_ptr<float>(), *sums = partial + tsmi_bn_partial_elems(ch);
       Tensor pg;
       if (op.norm.gamma >= 0) pg = at::empty({2 * ch}, w.options().requires_grad(false));
       Tensor dz, dconv = at::empty_like(c);
       if (op.residual >= 0 && op.relu) dz = at::empty_like(c);
-      {
-        std::lock_guard<std::mutex> own(g_scratch_lock);
-        check(tsmi_bn_backward(s, g.data_ptr(), c.data_ptr(),
-                               op.relu && op.residual >= 0 ? value[op.dst].data_ptr() : nullptr, n, ch, code, op.relu,
-                               op.norm.gamma >= 0 ? w.data_ptr() : nullptr, dtype_code(w), stats[i].data_ptr<float>(),
-                               partial, scratch_of(x, s).counters.data_ptr<int32_t>(), sums,
-                               pg.defined() ? pg.data_ptr() : nullptr, dz.defined() ? dz.data_ptr() : nullptr,
-                               dconv.data_ptr()));
-      }
+      check(tsmi_bn_backward(s, g.data_ptr(), c.data_ptr(),
+                             op.relu && op.residual >= 0 ? value[op.dst].data_ptr() : nullptr, n, ch, code, op.relu,
+                             op.norm.gamma >= 0 ? w.data_ptr() : nullptr, dtype_code(w), stats[i].data_ptr<float>(),
+                             partial, sums, pg.defined() ? pg.data_ptr() : nullptr,
+                             dz.defined() ? dz.data_ptr() : nullptr, dconv.data_ptr()));
       if (op.norm.gamma >= 0) result[1 + op.norm.gamma] = pg.narrow(0, ch, ch);
       if (op.norm.beta >= 0) result[1 + op.norm.beta] = pg.narrow(0, 0, ch);
       if (op.residual >= 0) {
@@ -537,7 +533,6 @@ Tensor train_stage(const std::shared_ptr<Stage> &stage, const Tensor &x, const s
         const Tensor work = floats(tsmi_bn_partial_elems(ch), x);
         node->stats[i] = floats(4 * ch, x);
         const Tensor &kind = nm.gamma >= 0 ? stage->params[nm.gamma] : nm.running_mean.defined() ? nm.running_mean : c;
-        std::lock_guard<std::mutex> own(g_scratch_lock);
         check(tsmi_bn_forward_train(
             s, c.data_ptr(), c.size(0), ch, code, nm.gamma >= 0 ? stage->params[nm.gamma].data_ptr() : nullptr,
             nm.beta >= 0 ? stage->params[nm.beta].data_ptr() : nullptr, dtype_code(kind),
@@ -545,7 +540,7 @@ Tensor train_stage(const std::shared_ptr<Stage> &stage, const Tensor &x, const s
             nm.running_var.defined() ? nm.running_var.data_ptr() : nullptr,
             nm.batches.defined() ? nm.batches.data_ptr<int64_t>() : nullptr, (float)nm.momentum, (float)nm.eps,
             op.residual >= 0 ? buf[op.residual].data_ptr() : nullptr, op.relu, work.data_ptr<float>(),
-            scratch_of(x, s).counters.data_ptr<int32_t>(), node->stats[i].data_ptr<float>(), y.data_ptr()));
+            node->stats[i].data_ptr<float>(), y.data_ptr()));
       }
       buf[op.dst] = y;
       if (record) node->conv_out[i] = op.has_norm ? c : Tensor();
