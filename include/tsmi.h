@@ -555,11 +555,15 @@ int tsmi_conv_fetch_on_demand(tsmi_stream_t s, const void *x, const void *w_pack
  * order of k, atomic free).  `products` holds K_vol * seg_rows * cout elements of the I/O
  * type, of which only the rows of existing pairs are touched.  tsmi_conv_segments_supported:
  * 1 for the shapes that have a variant (fp16 / bf16, K_vol <= 64, cin one of 128, 192, 256,
- * 384, cout a multiple of 8).  Same sums as conv_forward_implicit_gemm_cuda
+ * 384, cout a multiple of 8); tsmi_conv_segments_fit: the same with fp32 (cin a multiple of 32 from 64 to
+ * 384 but for 160, 224, 288 and 320 to 352, cout a multiple of 4).  tsmi_conv_segments_pay: 1 where this form is
+ * also the faster one (density: pairs per map entry).  Same sums as conv_forward_implicit_gemm_cuda
  * (convolution/convolution_forward_implicit_gemm_cuda.cu:1527-1986) with the per-offset
  * products rounded to the I/O type as conv_forward_fetch_on_demand_cuda's are
  * (convolution/convolution_forward_fetch_on_demand_cuda.cu:1981-2119). */
 int tsmi_conv_segments_supported(int kvol, int cin, int cout, int dtype);
+int tsmi_conv_segments_fit(int kvol, int cin, int cout, int dtype);
+int tsmi_conv_segments_pay(int64_t n_out, int kvol, int cin, int cout, int dtype, double density);
 int tsmi_pair_segments(tsmi_stream_t s, const int32_t *map, int64_t n_rows, int kvol,
                        int64_t seg_rows, int32_t *pool, int32_t *counts, int32_t *in_rows,
                        int32_t *pos);

@@ -287,3 +287,21 @@ def test_the_form_of_a_wide_layer_follows_the_measured_density_of_its_map(mods):
         taken, other = (plain, pair) if dense else (pair, plain)
         print(f"density {density:.3f}: pair form {pair:.1f} us, dense pass {plain:.1f} us")
         assert taken <= 1.15 * other, (density, pair, plain)
+
+
+@pytest.mark.parametrize("n,cin,cout", [(3000, 128, 128), (2100, 256, 256), (1301, 384, 256), (777, 192, 100),
+                                        (65, 96, 96), (64, 64, 132), (33, 384, 32), (1, 256, 128)])
+def test_fp32_convolution_over_segments_matches_oracle(mods, n, cin, cout):
+    """fp32 rows of 256 bytes to 1.5 KB (the last with tiles of 32 pairs), full and partial tiles and columns."""
+    backend, F = mods
+    rng = np.random.default_rng(n + cin + cout)
+    coords = random_coords(rng, n, (22, 18, 12))
+    omap_np = oracle.kmap_subm(coords, 3)
+    x = rng.standard_normal((n, cin)).astype(np.float32)
+    w = (rng.uniform(-1, 1, (27, cin, cout)) / np.sqrt(cin * 27)).astype(np.float32)
+    assert backend._C.tsmi_conv_segments_fit(27, cin, cout, 0) == 1
+    bias = rng.standard_normal(cout).astype(np.float32)
+    tx, tw, tb = (torch.from_numpy(a).cuda() for a in (x, w, bias))
+    y = backend.conv_implicit_gemm_segments(tx, backend.pack_weights(tw), 27, cin, cout, dev(omap_np), n, tb, None, True)
+    want = np.maximum(oracle.conv_implicit_gemm(x, w, omap_np, n) + bias[None, :], 0)
+    assert rel_rms(_f32(y), want) < 1e-5

@@ -111,6 +111,8 @@ def _load():
         "tsmi_conv_fetch_on_demand": [_vp, _vp, _vp, _vp, _i64, _vp, _vp, _i64, _vp, _i64, _i32,
                                       _i32, _i32, _i32, _i32, _i32, _vp, _vp, _i32, _vp, _vp],
         "tsmi_conv_segments_supported": [_i32, _i32, _i32, _i32],
+        "tsmi_conv_segments_fit": [_i32, _i32, _i32, _i32],
+        "tsmi_conv_segments_pay": [_i64, _i32, _i32, _i32, _i32, ctypes.c_double],
         "tsmi_pair_segments": [_vp, _vp, _i64, _i32, _i64, _vp, _vp, _vp, _vp],
         "tsmi_pair_segments_batch": [_vp, _i32, _vp],
         "tsmi_conv_implicit_gemm_segments": [_vp, _vp, _vp, _vp, _vp, _vp, _i64, _i64, _i32, _i32, _i32,
@@ -163,7 +165,7 @@ class _Library:
     _ASIS = ("tsmi_conv_implicit_gemm_packed", "tsmi_conv_implicit_gemm_segments_packed",
              "tsmi_conv_implicit_gemm_grouped_packed", "tsmi_last_error", "tsmi_version",
              "tsmi_host_voxelize")
-    _ASIS_ENDINGS = ("_elems", "_words", "_supported", "_bytes", "_capacity", "_padded")
+    _ASIS_ENDINGS = ("_elems", "_words", "_supported", "_fit", "_pay", "_bytes", "_capacity", "_padded")
 
     def __init__(self, lib):
         self._lib = lib
@@ -2072,11 +2074,6 @@ def _workspace_elems(n_out: int, kvol: int, cin: int, cout: int, code: int) -> i
     return _C.tsmi_conv_workspace_elems(n_out, n_out, kvol, 1, cin, cout, code, 0)
 
 
-@functools.lru_cache(maxsize=4096)
-def _segments_supported(kvol: int, cin: int, cout: int, code: int) -> bool:
-    return bool(_C.tsmi_conv_segments_supported(kvol, cin, cout, code))
-
-
 _TILE_COUNTERS = {}
 _N_TILE_COUNTERS = 4096
 
@@ -2414,9 +2411,10 @@ def hint_sparse_map(out_in_map: torch.Tensor) -> None:
 
 
 def _segments_pay(x, kvol, cin, cout, num_out_feats, out_in_map=None, force=None) -> bool:
-    """Whether a layer runs over pair segments: 16-bit features, a 3^3 or larger kernel, few rows
-    and many channels (the regime in which the dense pass is bound by the weight slabs it streams
-    per row tile) and a map with few pairs per row.  The cost of the pair form grows with the
+    """Whether a layer runs over pair segments: a 3^3 or larger kernel, the sizes of
+    tsmi_conv_segments_pay (16-bit features: few rows and many channels, the regime in which the dense
+    pass is bound by the weight slabs it streams per row tile; fp32: many channels, where it is bound by
+    the multiplications) and a map with few pairs per row.  The cost of the pair form grows with the
     number of pairs (every product row crosses memory twice), the dense pass keeps its sums in
     registers: measured on the levels of an 89,834-voxel scan (24 % of the map entries are pairs):
     8,045 rows 256 -> 256 32 vs 43 us, 384 -> 256 39 vs 57, 19,815 rows 128 -> 128 30 vs 36,
@@ -2432,19 +2430,26 @@ def _segments_pay(x, kvol, cin, cout, num_out_feats, out_in_map=None, force=None
     mode = igemm_through_segments
     if force is not None:  # a layer's own configuration (conv_config "pair_segments") decides
         mode = "always" if force else False
-    if not mode or not (kvol >= 27 and 0 < num_out_feats < 65536 and cout >= 128
-                        and (cin * cout > 128 * 128 or num_out_feats >= 12000)
-                        and _segments_supported(kvol, cin, cout, _dtype_code(x))):
+    if not mode:
         return False
-    if mode == "always":
-        return True
-    if out_in_map is None:
-        return False
-    density = map_density(out_in_map)  # measured, where the map's build counted its pairs
-    if density is not None:
-        return density <= segments_max_density
-    hit = _sparse_maps.get(id(out_in_map))
-    return hit is not None and hit() is out_in_map
+    code, density = _dtype_code(x), 0.0
+    if mode is True:
+        if out_in_map is None:
+            return False
+        density = known_density(out_in_map)
+        if density is None or (code != F32 and density > segments_max_density):
+            return False
+    return bool(_C.tsmi_conv_segments_pay(num_out_feats, kvol, cin, cout, code, density))
+
+
+def known_density(out_in_map) -> Optional[float]:
+    """Pairs per entry of a map: measured (map_density), or what a map hinted to be sparse has at most."""
+    density = map_density(out_in_map)
+    if density is None:
+        hit = _sparse_maps.get(id(out_in_map))
+        if hit is not None and hit() is out_in_map:
+            return segments_max_density
+    return density
 
 
 def conv_implicit_gemm_segments(x, wp, kvol, cin, cout, out_in_map, num_out_feats, bias=None,
@@ -2530,16 +2535,20 @@ def native_identity(n: int):
     return native().KernelMap(1, n, n, True, None, None)
 
 
-def native_segments(handle, x, channels, kmap, force) -> bool:
+def native_segments(handle, x, channels, kmap, force, coarse=None) -> bool:
     """Whether layers of a submanifold or strided map run over its pair segments, given the channels
-    of one that could (kernel volume, inputs, outputs); attaches the segments to the map's handle."""
+    of one that could (kernel volume, inputs, outputs); attaches the segments to the map's handle.
+    ``coarse``: the rows of the level below, where there is one."""
     if handle.has_segments:
         return True
     omap, n = kmap["out_in_map"], kmap["sizes"][1]
-    if n >= 65536 or not _segments_pay(x, *channels, n, omap, force):
+    if coarse is not None and kmap["subm"] and (level_thinning(coarse) or 0) >= 0.3:
+        hint_sparse_map(omap)  # (rows that thin out like a surface from here on)
+    if not _segments_pay(x, *channels, n, omap, force):
         return False
     seg = pair_segments(omap, n)
-    handle.set_segments(seg.buffer, seg.in_rows_ptr, seg.counts_ptr, seg.pos_ptr, seg.seg_rows)
+    handle.set_segments(seg.buffer, seg.in_rows_ptr, seg.counts_ptr, seg.pos_ptr, seg.seg_rows,
+                        known_density(omap) or 0.0)
     return True
 
 

@@ -251,8 +251,30 @@ extern "C" int tsmi_conv_fetch_on_demand(tsmi_stream_t s, const void *x, const v
 
 extern "C" int tsmi_conv_segments_supported(int kvol, int cin, int cout, int dtype) {
   const ConvOps *ops = ops_for(dtype);
-  if (!ops || kvol < 1 || cin < 1 || cout < 1) return 0;
-  return ops->segments_supported(kvol, cin, cout);
+  if (!ops || dtype == TSMI_F32 || kvol < 1 || cin < 1 || cout < 1) return 0;
+  return ops->segments_fit(kvol, cin, cout);
+}
+
+extern "C" int tsmi_conv_segments_fit(int kvol, int cin, int cout, int dtype) {
+  const ConvOps *ops = ops_for(dtype);
+  return ops && kvol >= 1 && cin >= 1 && cout >= 1 ? ops->segments_fit(kvol, cin, cout) : 0;
+}
+
+// Where the pair form is the faster one (density: pairs per entry of the map, about 0.2 for a scan).
+// 16-bit types: few rows and many channels, where the dense pass is bound by the weights it streams per row tile;
+// the pair form writes and reads a product row per pair.  (Its callers ask for a density of at most 0.35.)
+// fp32: the dense pass multiplies the whole map at a sixteenth of the 16-bit rate and is bound by that from 96
+// channels on, at any number of rows.  27 offsets, dense -> pairs, in us: density 0.22, 40k rows 64 -> 128
+// 155 -> 94, 128 -> 128 295 -> 129, 256 -> 256 1064 -> 349; 900 rows 96 -> 96 34 -> 23, 256 -> 256 50 -> 32;
+// density 0.45, 3.4k rows 128 -> 128 43 -> 45, 192 -> 128 59 -> 48, 256 -> 256 133 -> 83.  The products are kept
+// below 4 GiB.
+extern "C" int tsmi_conv_segments_pay(int64_t n_out, int kvol, int cin, int cout, int dtype, double density) {
+  if (n_out < 1 || kvol < 27 || !tsmi_conv_segments_fit(kvol, cin, cout, dtype)) return 0;
+  const int64_t work = (int64_t)cin * cout;
+  if (dtype != TSMI_F32)
+    return n_out < 65536 && cout >= 128 && (work > 128 * 128 || n_out >= 12000);
+  return (work >= 96 * 96 || (work >= 64 * 128 && n_out >= 12000)) && density <= (work >= 192 * 128 ? 0.5 : 0.35) &&
+         (n_out + 63) / 64 * 64 * kvol * cout * 4 <= ((int64_t)1 << 32);
 }
 
 static int implicit_gemm_segments(tsmi_stream_t s, const void *x, const void *w_packed,

@@ -65,7 +65,7 @@ struct ConvOps {
                      const int32_t *seg_steps, int64_t pair_cap, int x_col, int kvol, int cin,
                      int cout, int64_t identity, float *partial, int64_t partial_elems, void *dw);
   // 1 when `segments` has a variant for the shape
-  int (*segments_supported)(int kvol, int cin, int cout);
+  int (*segments_fit)(int kvol, int cin, int cout);
   // products[k * seg_rows + j, :] = X[in_rows[k * seg_rows + j], :] W[k] for j < counts[k]
   int (*segments)(hipStream_t s, const void *x, const void *wp, const int32_t *in_rows,
                   const int32_t *counts, int64_t seg_rows, int kvol, int cin, int cout, int mirrored,

@@ -98,6 +98,7 @@ struct KernelMap {
   // pair segments of `map` (tsmi_pair_segments), where its layers are to run over them
   Tensor segments;
   int64_t seg_in = 0, seg_counts = 0, seg_pos = 0, seg_rows = 0;
+  double density = 0;  // pairs per entry as far as it is known
   // grouped copy of `map` (tsmi_map_group_rows)
   Tensor grouped;
   std::vector<int64_t> grouped_at;
@@ -211,8 +212,8 @@ Tensor convolve(KernelMap &m, bool transposed, bool backward, const Tensor &x, c
     return y;
   }
   const bool own_map = !to_inputs || mirrored;
-  if (own_map && rules.segments && m.segments.defined() && c.n_out < 65536 && cout >= 128 &&
-      (cin * cout > 128 * 128 || c.n_out >= 12000) && tsmi_conv_segments_supported(m.kvol, cin, cout, c.dtype)) {
+  if (own_map && rules.segments && m.segments.defined() &&
+      tsmi_conv_segments_pay(c.n_out, m.kvol, cin, cout, c.dtype, m.density)) {
     c.in_rows = (const int32_t *)m.seg_in;
     c.counts = (const int32_t *)m.seg_counts;
     c.pos = (const int32_t *)m.seg_pos;
@@ -591,7 +592,8 @@ PYBIND11_MODULE(_native, mod) {
       .def_property_readonly("has_segments", [](const KernelMap &m) { return m.segments.defined(); })
       .def_property_readonly("has_grouped", [](const KernelMap &m) { return m.grouped.defined(); })
       .def("set_segments",
-           [](KernelMap &m, Tensor buffer, int64_t in, int64_t counts, int64_t pos, int64_t rows) {
+           [](KernelMap &m, Tensor buffer, int64_t in, int64_t counts, int64_t pos, int64_t rows, double density) {
+             m.density = density;
              m.segments = std::move(buffer);
              m.seg_in = in, m.seg_counts = counts, m.seg_pos = pos, m.seg_rows = rows;
            })

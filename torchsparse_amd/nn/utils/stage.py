@@ -104,13 +104,14 @@ class _Builder:
         elif stride != (1, 1, 1):
             after = self.level + 1
         slot = (self.level, after, conv.kernel_size, stride, dilation, conv.transposed, conv.padding, pointwise)
-        wide = conv.out_channels >= 128
+        wide = conv.out_channels >= 128 or kernel.dtype == torch.float32
         at = next((i for i, s in enumerate(self.slots) if s[0] == slot), None)
         if at is None:
             at = len(self.slots)
             self.slots.append([slot, None, 0])
         if not pointwise and conv.kernel_volume >= 27:
-            if wide and self.slots[at][1] is None:  # (channels by which a map's form is decided)
+            most = self.slots[at][1]  # (channels by which a map's form is decided)
+            if wide and (most is None or conv.in_channels * conv.out_channels > most[1] * most[2]):
                 self.slots[at][1] = (conv.kernel_volume, conv.in_channels, conv.out_channels)
             self.slots[at][2] += 1
         self.level = after
@@ -331,7 +332,8 @@ def run(owner: nn.Module, x: SparseTensor, modules: Optional[Tuple[nn.Module, ..
         dict.setdefault(kmap, "kernel_size", kernel_size)
         handle = _native_map(backend, kmap, transposed)
         if wide is not None and not transposed:
-            segments = backend.native_segments(handle, feats, wide, kmap, force) or segments
+            coarse = levels.get(tuple(2 * s for s in here))
+            segments = backend.native_segments(handle, feats, wide, kmap, force, coarse and coarse[0]) or segments
         if uses and not training and not transposed:
             backend.native_grouped(handle, kmap, uses)
         maps.append(handle)
