@@ -397,6 +397,10 @@ int64_t tsmi_packed_weight_elems(int kvol, int cin, int cout);
  * No counterpart in the reference (its kernels read [K_vol,Cin,Cout] directly). */
 int tsmi_pack_weights(tsmi_stream_t s, const void *w, void *w_packed, int kvol, int cin,
                       int cout, int dtype);
+/* The same layout for a layer Cin -> Cout whose kernel is given as [K_vol, Cout, Cin] (the input gradient's of one
+ * Cout -> Cin). */
+int tsmi_pack_weights_turned(tsmi_stream_t s, const void *w, void *w_packed, int kvol, int cin,
+                             int cout, int dtype);
 /* The same for n tensors of one type in one launch (48 at a time); shapes: n rows (K_vol, Cin, Cout). */
 int tsmi_pack_weights_many(tsmi_stream_t s, const void *const *w, void *const *w_packed,
                            const int32_t *shapes, int n, int dtype);
@@ -780,6 +784,10 @@ int tsmi_devoxelize_forward(tsmi_stream_t s, const void *feat, const int32_t *in
 int tsmi_devoxelize_backward(tsmi_stream_t s, const void *top_grad, const float *weight,
                              const int32_t *order, const int32_t *starts, int64_t n, int64_t n_vox,
                              int c, int dtype, void *bottom_grad);
+
+/* y[i, :c] = x[i, :], y[i, c:] = 0: rows of c elements of `dtype` laid out c_pad apart, c_pad the next multiple of 16
+ * bytes' worth (y 16-byte aligned). */
+int tsmi_pad_columns(tsmi_stream_t s, const void *x, int64_t n, int c, int dtype, void *y);
 
 /* dense[b,x,y,z,:] = feats[i,:] for coords[i] = (b,x,y,z) inside spatial_range (HOST int32[4],
  * extents B,X,Y,Z); the caller clears `dense` first.  The backward copies the other way

@@ -195,3 +195,27 @@ def test_changed_weights_replaced_parameters_and_hooks(mods):
     net.float()
     feats = feats.float()
     check()
+
+
+@pytest.mark.parametrize("cin,cout,kernel,stride,n,dtype,tol", [
+    (23, 45, 3, 1, 3000, torch.float32, 2e-5), (3, 1, 3, 1, 700, torch.float32, 2e-5), (9, 7, 2, 2, 129, torch.float16, 2e-2),
+    (5, 33, 3, 2, 4000, torch.bfloat16, 8e-2), (64, 96, 3, 1, 5000, torch.float16, 2e-2), (1, 17, 5, 1, 65, torch.float16, 2e-2)])
+def test_a_layer_on_its_own(mods, cin, cout, kernel, stride, n, dtype, tol, monkeypatch):
+    """Rows that are not whole 16-byte pieces, forward and both gradients; the result may be written over."""
+    ts, spnn, _, _, stage, _ = mods
+    torch.manual_seed(n)
+    coords = cloud(n, max(int((4 * n) ** (1 / 3)), 8), n)
+    layer = spnn.Conv3d(cin, cout, kernel, stride=stride, padding=1).cuda().to(dtype).train()
+    feats = torch.randn(n, cin, device="cuda").to(dtype)
+
+    def step():
+        x = feats.clone().requires_grad_()
+        layer.zero_grad(set_to_none=True)
+        y = layer(ts.SparseTensor(x, coords)).feats
+        out = y.detach().clone()
+        y.mul_(2)
+        y.backward(torch.cos(torch.arange(y.numel(), device="cuda").view_as(y)).to(dtype))
+        return {"y": out, "dx": x.grad, "dw": layer.kernel.grad}
+    one, two, calls = both(stage, step, monkeypatch)
+    assert calls == 1
+    _close(one, two, tol)

@@ -137,6 +137,7 @@ def _load():
         "tsmi_voxelize_backward": [_vp, _vp, _vp, _vp, _i64, _i32, _i64, _i32, _vp],
         "tsmi_devoxelize_forward": [_vp, _vp, _vp, _vp, _i64, _i64, _i32, _i32, _vp],
         "tsmi_devoxelize_backward": [_vp, _vp, _vp, _vp, _vp, _i64, _i64, _i32, _i32, _vp],
+        "tsmi_pad_columns": [_vp, _vp, _i64, _i32, _i32, _vp],
         "tsmi_to_dense_forward": [_vp, _vp, _vp, _i64, _i32, _I4, _i32, _vp],
         "tsmi_to_dense_backward": [_vp, _vp, _vp, _i64, _i32, _I4, _i32, _vp],
         "tsmi_bn_forward_train": [_vp, _vp, _i64, _i32, _i32, _vp, _vp, _i32, _vp, _vp, _vp, _f32, _f32, _vp,
@@ -2093,6 +2094,16 @@ def _tile_counters(device, stream: int):
     return t
 
 
+def whole_pieces(x: torch.Tensor) -> torch.Tensor:
+    """Rows of ``x`` [N, C] in whole 16-byte pieces: x itself, or a copy with zero columns appended."""
+    c, per = x.shape[1], 16 // x.element_size()
+    if c % per == 0:
+        return x
+    y = x.new_empty(x.shape[0], (c + per - 1) // per * per)
+    _check(_C.tsmi_pad_columns(_stream(), _ptr(x), x.shape[0], c, _dtype_code(x), _ptr(y)))
+    return y
+
+
 def conv_forward_implicit_gemm_cuda(in_feats, kernel, out_in_map, num_out_feats, num_out_channels,
                                     allow_tf32=False, allow_fp16=True, bias=None, residual=None,
                                     relu=False, segments=None) -> torch.Tensor:
@@ -2482,6 +2493,11 @@ def _implicit_gemm(x, wp, kvol, cin, cout, out_in_map, num_out_feats, bias=None,
     """``out`` / ``also``: the result goes into ``out`` instead of a new tensor, and a second time
     into ``also`` (see _placed: column slices of wider buffers, which spares the copy of a later
     concatenation)."""
+    if (cin * x.element_size()) % 16 and not (cin <= 8 and x.element_size() == 2):
+        # the kernels that load rows in 16-byte pieces (the packed weights are padded already); 16-bit layers
+        # of up to 8 channels have one that takes any number
+        x = whole_pieces(x)
+        cin = x.shape[1]
     if _segments_pay(x, kvol, cin, cout, num_out_feats, out_in_map, segments):
         return conv_implicit_gemm_segments(x, wp, kvol, cin, cout, out_in_map, num_out_feats, bias,
                                            residual, relu, out, also)

@@ -39,7 +39,16 @@ extern "C" int tsmi_pack_weights(tsmi_stream_t s, const void *w, void *w_packed,
   const ConvOps *ops = ops_for(dtype);
   if (int e = check_shapes("pack_weights", ops, kvol, cin, cout)) return e;
   TSMI_REQUIRE(w && w_packed, "pack_weights: null pointer");
-  const PackJob job{w, w_packed, kvol, cin, cout};
+  const PackJob job{w, w_packed, kvol, cin, cout, 0};
+  return ops->pack((hipStream_t)s, &job, 1);
+}
+
+extern "C" int tsmi_pack_weights_turned(tsmi_stream_t s, const void *w, void *w_packed, int kvol, int cin,
+                                        int cout, int dtype) {
+  const ConvOps *ops = ops_for(dtype);
+  if (int e = check_shapes("pack_weights_turned", ops, kvol, cin, cout)) return e;
+  TSMI_REQUIRE(w && w_packed, "pack_weights_turned: null pointer");
+  const PackJob job{w, w_packed, kvol, cin, cout, 1};
   return ops->pack((hipStream_t)s, &job, 1);
 }
 
@@ -51,7 +60,7 @@ extern "C" int tsmi_pack_weights_many(tsmi_stream_t s, const void *const *w, voi
   for (int i = 0; i < n; ++i) {
     if (int e = check_shapes("pack_weights_many", ops, shapes[3 * i], shapes[3 * i + 1], shapes[3 * i + 2])) return e;
     TSMI_REQUIRE(w[i] && w_packed[i], "pack_weights_many: null pointer");
-    jobs[i] = PackJob{w[i], w_packed[i], shapes[3 * i], shapes[3 * i + 1], shapes[3 * i + 2]};
+    jobs[i] = PackJob{w[i], w_packed[i], shapes[3 * i], shapes[3 * i + 1], shapes[3 * i + 2], 0};
   }
   return n == 0 ? TSMI_OK : ops->pack((hipStream_t)s, jobs.data(), n);
 }

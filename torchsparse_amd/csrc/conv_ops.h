@@ -26,6 +26,7 @@ struct PackJob {
   const void *w;
   void *wp;
   int kvol, cin, cout;
+  int turned;  // w is [K_vol, Cout, Cin]
 };
 
 struct ConvOps {

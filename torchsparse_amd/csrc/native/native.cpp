@@ -55,6 +55,15 @@ int dtype_code(const Tensor &t) {
 
 int64_t ceil128(int64_t n) { return (n + 127) / 128 * 128; }
 
+// Rows of x in whole 16-byte pieces (what the fast kernels load): with zero columns appended where they are not.
+Tensor whole_pieces(const Tensor &x) {
+  const int64_t per = 16 / x.element_size(), c = x.size(1);
+  if (c % per == 0) return x;
+  Tensor y = at::empty({x.size(0), (c + per - 1) / per * per}, x.options());
+  check(tsmi_pad_columns(stream_of(x), x.data_ptr(), x.size(0), (int)c, dtype_code(x), y.data_ptr()));
+  return y;
+}
+
 Tensor ints(int64_t n, const Tensor &like) { return at::empty({n}, like.options().dtype(at::kInt)); }
 Tensor floats(int64_t n, const Tensor &like) { return at::empty({n}, like.options().dtype(at::kFloat)); }
 
@@ -168,10 +177,19 @@ void make(const tsmi_conv_call &c, Pending *pending) {
 
 // y (rows of `map`, or with `backward` of its transposed direction) = act(conv(x) + bias + residual).
 // `w`: packed weights, the reduction axis contiguous.
-Tensor convolve(KernelMap &m, bool transposed, bool backward, const Tensor &x, const void *w, int cin, int cout,
+Tensor convolve(KernelMap &m, bool transposed, bool backward, const Tensor &x0, const void *w, int cin, int cout,
                 const Tensor &bias, const Tensor &residual, bool relu, const Rules &rules, const Place *out,
                 const Place *also, Pending *pending = nullptr) {
   tsmi_conv_call c{};
+  Tensor x = x0;
+  cin = (int)x.size(1);  // (a gradient may come in whole pieces)
+  // (16-bit layers of up to 8 channels have a kernel that takes any number; packed weights are padded already)
+  if (cin * x.element_size() % 16 != 0 && !(x.element_size() == 2 && cin <= 8)) {
+    if (pending) check(tsmi_launch_thread_flush());
+    x = whole_pieces(x0);
+    cin = (int)x.size(1);
+    if (pending) pending->tensors.push_back(x);
+  }
   c.stream = stream_of(x);
   c.x = x.data_ptr();
   c.w_packed = w;
@@ -290,6 +308,9 @@ struct Stage {
   std::vector<Packed> packed;  // per operation
   int buffers = 1;
 
+  // Whether the backward reads the last result (the caller may write over it otherwise): a residual layer's mask.
+  bool needs_output() const { return ops.back().has_norm && ops.back().relu && ops.back().residual >= 0; }
+
   void fits(const Tensor &x, const std::vector<Map> &maps) const {
     TORCH_CHECK(!ops.empty() && x.dim() == 2 && x.is_contiguous() && x.size(1) == ops[0].cin, "stage: another input");
     for (const Op &op : ops) {
@@ -364,15 +385,9 @@ struct Stage {
   }
 };
 
-// Rows of x with zero columns appended up to whole 16-byte pieces.
-Tensor pad_columns(const Tensor &x) {
-  const int64_t per = 16 / x.element_size(), extra = (per - x.size(1) % per) % per;
-  return extra == 0 ? x : at::constant_pad_nd(x, {0, extra});
-}
-
 // dW [kvol, cin, cout] of a convolution from its input and its output's gradient.
 Tensor weight_grad(KernelMap &m, bool transposed, const Tensor &x0, const Tensor &dy0, int cin, int cout) {
-  const Tensor x = pad_columns(x0), dy = pad_columns(dy0);
+  const Tensor x = whole_pieces(x0), dy = whole_pieces(dy0);
   const int ci = (int)x.size(1), co = (int)dy.size(1), code = dtype_code(x);
   const tsmi_stream_t s = stream_of(x);
   Tensor dw = at::empty({m.kvol, ci, co}, x.options());
@@ -402,10 +417,9 @@ Tensor input_grad(KernelMap &m, bool transposed, const Tensor &dy, const Tensor 
   const void *w = weight.data_ptr();
   Tensor packed;
   if (tsmi_packed_weight_elems(m.kvol, cout, cin) != weight.numel()) {
-    const Tensor turned = weight.detach().view({m.kvol, cin, cout}).transpose(1, 2).contiguous();
-    packed = at::empty({tsmi_packed_weight_elems(m.kvol, cout, cin)}, turned.options());
-    check(tsmi_pack_weights(stream_of(dy), turned.data_ptr(), packed.data_ptr(), m.kvol, cout, cin,
-                            dtype_code(dy)));
+    packed = at::empty({tsmi_packed_weight_elems(m.kvol, cout, cin)}, weight.options().requires_grad(false));
+    check(tsmi_pack_weights_turned(stream_of(dy), weight.data_ptr(), packed.data_ptr(), m.kvol, cout, cin,
+                                   dtype_code(dy)));
     w = packed.data_ptr();
   }
   return convolve(m, transposed, true, dy, w, cout, cin, Tensor(), more, false, rules, nullptr, nullptr);
@@ -450,7 +464,7 @@ torch::autograd::variable_list StageNode::apply(torch::autograd::variable_list &
   at::AutoDispatchBelowADInplaceOrView below;
   std::vector<Tensor> value = buf, weights(n_params);
   value[0] = input.unpack();
-  value[ops.back().dst] = output.unpack(shared_from_this());
+  if (stage->needs_output()) value[ops.back().dst] = output.unpack(shared_from_this());
   for (size_t i = 0; i < n_params; ++i) weights[i] = params[i].unpack();
   std::vector<Tensor> grad(stage->buffers);
   Tensor top = grads[0].contiguous();
@@ -490,6 +504,7 @@ torch::autograd::variable_list StageNode::apply(torch::autograd::variable_list &
       }
       g = dconv;
     }
+    if (g.size(1) * g.element_size() % 16 != 0) g = whole_pieces(g);  // (once for both gradients)
     if (task_should_compute_output(1 + op.weight)) {
       Tensor dw = weight_grad(m, op.transposed, value[op.src], g, op.cin, op.cout);
       result[1 + op.weight] = dw.view(weights[op.weight].sizes());
@@ -556,7 +571,7 @@ Tensor train_stage(const std::shared_ptr<Stage> &stage, const Tensor &x, const s
     node->input = torch::autograd::SavedVariable(x, false);
     for (const Tensor &p : stage->params) node->params.emplace_back(p, false);
     torch::autograd::set_history(y, node);
-    node->output = torch::autograd::SavedVariable(y, true);
+    if (stage->needs_output()) node->output = torch::autograd::SavedVariable(y, true);
   }
   return y;
 }

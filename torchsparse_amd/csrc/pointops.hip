@@ -385,6 +385,20 @@ inline int vec_width(int c, std::initializer_list<const void *> ptrs) {
   return v;
 }
 
+// Rows of c elements laid out in whole 16-byte pieces: a thread makes one piece.
+template <typename T>
+__global__ __launch_bounds__(256) void pad_columns_kernel(const T *x, int64_t n, int c, int pieces, uint4 *y) {
+  constexpr int kPer = 16 / (int)sizeof(T);
+  const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
+  if (i >= n * pieces) return;
+  const int64_t r = i / pieces;
+  const int first = (int)(i - r * pieces) * kPer;
+  alignas(16) T v[kPer];
+#pragma unroll
+  for (int e = 0; e < kPer; ++e) v[e] = first + e < c ? x[r * c + first + e] : T{0};
+  y[i] = *(const uint4 *)v;
+}
+
 }  // namespace
 }  // namespace tsmi
 
@@ -636,4 +650,20 @@ extern "C" int tsmi_to_dense_backward(tsmi_stream_t s, const void *top_grad, con
   TSMI_BY_DTYPE(dtype, return (dense_copy_t<T, false>((hipStream_t)s, bottom_grad, coords, n, c,
                                                       spatial_range, (void *)top_grad)));
   return TSMI_OK;
+}
+
+extern "C" int tsmi_pad_columns(tsmi_stream_t s, const void *x, int64_t n, int c, int dtype, void *y) {
+  TSMI_REQUIRE(n >= 0 && c >= 1, "pad_columns: bad arguments");
+  if (n == 0) return TSMI_OK;
+  TSMI_REQUIRE(x && y && aligned16(y), "pad_columns: null or misaligned pointer");
+  const int per = dtype == TSMI_F32 ? 4 : 8, pieces = (c + per - 1) / per;
+  TSMI_GRID_CHECK(n * pieces);
+  const dim3 grid((unsigned)ceil_div(n * pieces, 256));
+  if (dtype == TSMI_F32)
+    hipLaunchKernelGGL(pad_columns_kernel<uint32_t>, grid, dim3(256), 0, (hipStream_t)s, (const uint32_t *)x, n, c,
+                       pieces, (uint4 *)y);
+  else  // (bits are moved, whatever the 16-bit type)
+    hipLaunchKernelGGL(pad_columns_kernel<uint16_t>, grid, dim3(256), 0, (hipStream_t)s, (const uint16_t *)x, n, c,
+                       pieces, (uint4 *)y);
+  return check_launch("pad_columns_kernel");
 }

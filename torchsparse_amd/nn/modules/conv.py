@@ -83,6 +83,11 @@ class Conv3d(nn.Module):
                                    dilation, self.transposed, self._config, residual, self.activation, out, also)
             if done is not None:
                 return done
+        elif self.training and residual is None and out is None and also is None and torch.is_grad_enabled():
+            from ..utils import stage
+            done = stage.run(self, input)  # (one autograd node, made natively)
+            if done is not None:
+                return done
         return F.conv3d(input, weight=self.kernel, kernel_size=self.kernel_size, bias=self.bias,
                         stride=self.stride, padding=self.padding, dilation=self.dilation,
                         transposed=self.transposed, generative=self.generative,

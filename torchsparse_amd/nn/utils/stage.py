@@ -38,7 +38,7 @@ class _Unfit(Exception):
 
 
 class _Plan:
-    __slots__ = ("native", "slots", "modules", "members", "training", "cin", "first", "lead", "out_level")
+    __slots__ = ("native", "slots", "modules", "members", "training", "cin", "lead", "out_level", "config")
 
     def current(self) -> bool:
         """Whether the modules still are what the plan was compiled from: the same parameters and buffers, no hooks."""
@@ -65,7 +65,7 @@ class _Builder:
         self.training = training
         self.ops, self.params, self.slots, self.modules, self.members = [], [], [], [], []
         self.index = {}
-        self.buffers, self.level, self.dtype = 1, 0, None
+        self.buffers, self.level, self.config = 1, 0, None
 
     def param(self, module, name) -> int:
         value = module._parameters[name]
@@ -84,8 +84,9 @@ class _Builder:
 
     def conv(self, conv, src: int, norm=None, relu: bool = False, residual: int = -1) -> int:
         """Appends act(norm(conv(src)) + residual); returns the buffer of the result."""
-        if type(conv) is not self.Conv3d or conv.generative or conv._config is not None:
+        if type(conv) is not self.Conv3d or conv.generative or (self.ops and conv._config is not self.config):
             raise _Unfit
+        self.config = conv._config
         self.see(conv)
         kernel = conv._parameters["kernel"]
         if conv.activation not in (None, "relu") or (self.training and (conv.activation or conv.bias is not None)):
@@ -227,6 +228,7 @@ class _Builder:
         plan.lead = self.params[0]
         plan.cin = self.ops[0][0][9]
         plan.out_level = self.level
+        plan.config = self.config
         return plan
 
 
@@ -234,6 +236,8 @@ def _compile(modules: Tuple[nn.Module, ...], training: bool) -> Optional[_Plan]:
     try:
         b = _Builder(training)
         out = 0
+        if training and len(modules) == 1 and type(modules[0]) is b.Conv3d:
+            return b.finish(b.conv(modules[0], 0))  # (a layer on its own needs no norm behind it)
         for m in modules:
             out = b.module(m, out)
         return b.finish(out)
@@ -293,7 +297,7 @@ def run(owner: nn.Module, x: SparseTensor, modules: Optional[Tuple[nn.Module, ..
         return None
     if feats.shape[1] != plan.cin or feats.shape[0] < (2 if training else 1):
         return None
-    config = _cfg.get_global_conv_config()
+    config = plan.config or _cfg.get_global_conv_config()
     if config is None:
         config = _cfg._shared_default_config(get_conv_mode())
     if config["dataflow"] != _cfg.Dataflow.ImplicitGEMM or config["ifsort"]:
@@ -334,8 +338,8 @@ def run(owner: nn.Module, x: SparseTensor, modules: Optional[Tuple[nn.Module, ..
         if wide is not None and not transposed:
             coarse = levels.get(tuple(2 * s for s in here))
             segments = backend.native_segments(handle, feats, wide, kmap, force, coarse and coarse[0]) or segments
-        if uses and not training and not transposed:
-            backend.native_grouped(handle, kmap, uses)
+        if uses and not transposed:  # (in training the input gradient of a submanifold layer is a second use)
+            backend.native_grouped(handle, kmap, 2 * uses if training and kmap["subm"] else uses)
         maps.append(handle)
     out_stride = strides[plan.out_level]
     out_coords, out_range = (x.coords, x.spatial_range) if plan.out_level == 0 else levels[out_stride]
