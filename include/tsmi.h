@@ -660,8 +660,12 @@ typedef struct {
   void *products;
   const int32_t *grouped, *row_of, *order64, *order128;
   int64_t n_grouped;
+  int64_t n_in;  // rows of x (0: not said; some kernels then do without)
 } tsmi_conv_call;
 int tsmi_conv(const tsmi_conv_call *call);
+/* 1 where a call over the map itself that gives n_in has the kernel for narrow layers (all weights in the LDS), which
+ * makes neither grouped rows nor an offset split worth having. */
+int tsmi_conv_streams(int kvol, int cin, int cout, int dtype);
 
 /* A launch thread for the convolution calls of a forward (no counterpart in the reference, whose
  * calls are made one by one from the interpreter's thread).  Between _open and _close the three

@@ -111,6 +111,7 @@ def _load():
         "tsmi_conv_fetch_on_demand": [_vp, _vp, _vp, _vp, _i64, _vp, _vp, _i64, _vp, _i64, _i32,
                                       _i32, _i32, _i32, _i32, _i32, _vp, _vp, _i32, _vp, _vp],
         "tsmi_conv_segments_supported": [_i32, _i32, _i32, _i32],
+        "tsmi_conv_streams": [_i32, _i32, _i32, _i32],
         "tsmi_conv_segments_fit": [_i32, _i32, _i32, _i32],
         "tsmi_conv_segments_pay": [_i64, _i32, _i32, _i32, _i32, ctypes.c_double],
         "tsmi_pair_segments": [_vp, _vp, _i64, _i32, _i64, _vp, _vp, _vp, _vp],
@@ -122,6 +123,7 @@ def _load():
         "tsmi_launch_thread_close": [],
         "tsmi_conv_implicit_gemm_packed": [ctypes.c_char_p],
         "tsmi_conv_implicit_gemm_segments_packed": [ctypes.c_char_p],
+        "tsmi_conv": [ctypes.c_char_p],
         "tsmi_conv_implicit_gemm_grouped_packed": [ctypes.c_char_p],
         "tsmi_conv_implicit_gemm_grouped": [_vp, _vp, _vp, _vp, _vp, _vp, _vp, _i64, _i64, _i32, _i32, _i32, _i32,
                                             _vp, _vp, _i32, _vp],
@@ -163,10 +165,10 @@ class _Library:
     convolution calls, which go to that thread inside a region, the thread's own entry points and
     the entry points that only answer a question are passed through as they are."""
 
-    _ASIS = ("tsmi_conv_implicit_gemm_packed", "tsmi_conv_implicit_gemm_segments_packed",
+    _ASIS = ("tsmi_conv", "tsmi_conv_implicit_gemm_packed", "tsmi_conv_implicit_gemm_segments_packed",
              "tsmi_conv_implicit_gemm_grouped_packed", "tsmi_last_error", "tsmi_version",
              "tsmi_host_voxelize")
-    _ASIS_ENDINGS = ("_elems", "_words", "_supported", "_fit", "_pay", "_bytes", "_capacity", "_padded")
+    _ASIS_ENDINGS = ("_elems", "_words", "_supported", "_fit", "_pay", "_streams", "_bytes", "_capacity", "_padded")
 
     def __init__(self, lib):
         self._lib = lib
@@ -1965,6 +1967,8 @@ def keep_pending(pending) -> None:
 
 _PACK20 = struct.Struct("20q").pack
 _PACK21 = struct.Struct("21q").pack
+_PACK_CONV = struct.Struct("9q6i18q").pack  # a tsmi_conv_call
+_NO_FORM = (0,) * 10                        # (its fields of the segment and grouped forms)
 
 
 class ColumnSlice:
@@ -2092,6 +2096,11 @@ def _tile_counters(device, stream: int):
     if _pin_sinks:
         _pin(t)
     return t
+
+
+@functools.lru_cache(maxsize=4096)
+def _streams(kvol: int, cin: int, cout: int, code: int) -> bool:
+    return bool(_C.tsmi_conv_streams(kvol, cin, cout, code))
 
 
 def whole_pieces(x: torch.Tensor) -> torch.Tensor:
@@ -2493,17 +2502,27 @@ def _implicit_gemm(x, wp, kvol, cin, cout, out_in_map, num_out_feats, bias=None,
     """``out`` / ``also``: the result goes into ``out`` instead of a new tensor, and a second time
     into ``also`` (see _placed: column slices of wider buffers, which spares the copy of a later
     concatenation)."""
-    if (cin * x.element_size()) % 16 and not (cin <= 8 and x.element_size() == 2):
+    if (cin * x.element_size()) % 16 and (cin > 8 or x.element_size() != 2 or (
+            x.shape[0] >= 131072 and _streams(kvol, 8, cout, _dtype_code(x)))):
         # the kernels that load rows in 16-byte pieces (the packed weights are padded already); 16-bit layers
-        # of up to 8 channels have one that takes any number
+        # of up to 8 channels have one that takes any number, which is the faster one over fewer rows
         x = whole_pieces(x)
         cin = x.shape[1]
     if _segments_pay(x, kvol, cin, cout, num_out_feats, out_in_map, segments):
         return conv_implicit_gemm_segments(x, wp, kvol, cin, cout, out_in_map, num_out_feats, bias,
                                            residual, relu, out, also)
     if _grouping_pays(x, kvol, cin, cout, num_out_feats, out_in_map):
+        if _streams(kvol, cin, cout, _dtype_code(x)):
+            # a narrow layer: its kernel has nothing to gain from the order (the wider ones over this map have)
+            grouped_map(out_in_map, num_out_feats)
+            return _dense_gemm(x, wp, kvol, cin, cout, out_in_map, num_out_feats, bias, residual, relu, out, also)
         return conv_implicit_gemm_grouped(x, wp, kvol, cin, cout, out_in_map, num_out_feats, bias,
                                           residual, relu, out, also)
+    return _dense_gemm(x, wp, kvol, cin, cout, out_in_map, num_out_feats, bias, residual, relu, out, also)
+
+
+def _dense_gemm(x, wp, kvol, cin, cout, out_in_map, num_out_feats, bias, residual, relu, out, also) -> torch.Tensor:
+    """... over the map as it is."""
     if out is None and also is None:
         y = x.new_empty(num_out_feats, cout)  # (the cheapest form of the call: 1.2 us against 1.6)
         at, ldy, a2, ld2 = y.data_ptr(), 0, 0, 0
@@ -2512,22 +2531,23 @@ def _implicit_gemm(x, wp, kvol, cin, cout, out_in_map, num_out_feats, bias=None,
     code = _dtype_code(x)
     stream = _stream()
     pb, pr = _epilogue_args(bias, residual, x, num_out_feats, cout)
-    # (the arguments of tsmi_conv_implicit_gemm in one block: one conversion instead of 18)
+    # (the arguments in one block: one conversion instead of 30)
     ws_elems = _workspace_elems(num_out_feats, kvol, cin, cout, code) if num_out_feats < 65536 else 0
     if ws_elems > 0:  # (only maps with few row tiles use the offset split)
         with _scratch_lock:
-            block = _PACK21(stream, x.data_ptr(), wp.data_ptr(), out_in_map.data_ptr(), out_in_map.shape[0],
-                            num_out_feats, kvol, cin, cout, code, pb or 0, pr or 0, int(relu),
-                            _scratch(x.device, stream, 4 * ws_elems), ws_elems,
-                            _tile_counters(x.device, stream).data_ptr(), _N_TILE_COUNTERS, at, ldy, a2, ld2)
-            if not (_region_depth and _hand_over(0, block, 21, (x, wp, out_in_map, bias, residual, y, also,
+            block = _PACK_CONV(stream, x.data_ptr(), wp.data_ptr(), at, a2, ldy, ld2, pb or 0, pr or 0, relu, code, kvol,
+                               cin, cout, 0, num_out_feats, out_in_map.shape[0], out_in_map.data_ptr(),
+                               _scratch(x.device, stream, 4 * ws_elems), ws_elems,
+                               _tile_counters(x.device, stream).data_ptr(), _N_TILE_COUNTERS, *_NO_FORM, x.shape[0])
+            if not (_region_depth and _hand_over(3, block, 30, (x, wp, out_in_map, bias, residual, y, also,
                                                                 _SCRATCH.get((x.device.index, stream))))):
-                _check(_C.tsmi_conv_implicit_gemm_packed(block))
+                _check(_C.tsmi_conv(block))
     else:
-        block = _PACK21(stream, x.data_ptr(), wp.data_ptr(), out_in_map.data_ptr(), out_in_map.shape[0], num_out_feats,
-                        kvol, cin, cout, code, pb or 0, pr or 0, int(relu), 0, 0, 0, _N_TILE_COUNTERS, at, ldy, a2, ld2)
-        if not (_region_depth and _hand_over(0, block, 21, (x, wp, out_in_map, bias, residual, y, also))):
-            _check(_C.tsmi_conv_implicit_gemm_packed(block))
+        block = _PACK_CONV(stream, x.data_ptr(), wp.data_ptr(), at, a2, ldy, ld2, pb or 0, pr or 0, relu, code, kvol, cin,
+                           cout, 0, num_out_feats, out_in_map.shape[0], out_in_map.data_ptr(), 0, 0, 0,
+                           _N_TILE_COUNTERS, *_NO_FORM, x.shape[0])
+        if not (_region_depth and _hand_over(3, block, 30, (x, wp, out_in_map, bias, residual, y, also))):
+            _check(_C.tsmi_conv(block))
     return y
 
 

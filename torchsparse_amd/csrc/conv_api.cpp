@@ -264,6 +264,11 @@ extern "C" int tsmi_conv_segments_supported(int kvol, int cin, int cout, int dty
   return ops->segments_fit(kvol, cin, cout);
 }
 
+extern "C" int tsmi_conv_streams(int kvol, int cin, int cout, int dtype) {
+  const ConvOps *ops = ops_for(dtype);
+  return ops && kvol >= 1 && cin >= 1 && cout >= 1 ? ops->streams(kvol, cin, cout) : 0;
+}
+
 extern "C" int tsmi_conv_segments_fit(int kvol, int cin, int cout, int dtype) {
   const ConvOps *ops = ops_for(dtype);
   return ops && kvol >= 1 && cin >= 1 && cout >= 1 ? ops->segments_fit(kvol, cin, cout) : 0;
@@ -405,7 +410,7 @@ extern "C" int tsmi_conv_implicit_gemm_segments_packed(const int64_t *a) {
 // One convolution in whichever form the caller has products of the map for.
 extern "C" int tsmi_conv(const tsmi_conv_call *c) {
   TSMI_REQUIRE(c, "conv: null call");
-  OutPlace place{c->ldy, c->y2, c->ldy2, c->mirrored};
+  OutPlace place{c->ldy, c->y2, c->ldy2, c->mirrored, c->n_in};
   if (c->in_rows)
     return implicit_gemm_segments(c->stream, c->x, c->w_packed, c->in_rows, c->counts, c->pos, c->seg_rows, c->n_out,
                                   c->kvol, c->cin, c->cout, c->dtype, c->bias, c->residual, c->relu, c->products,

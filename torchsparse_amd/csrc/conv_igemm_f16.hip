@@ -35,6 +35,7 @@ struct TraitsF16 {
 #include "conv_small_cin.inc"
 #include "conv_tile.inc"
 #include "conv_igemm2.inc"
+#include "conv_stream.inc"
 #include "conv_segments.inc"
 #include "conv_plan.inc"
 #include "conv_wgrad.inc"

@@ -19,6 +19,7 @@ struct OutPlace {
   void *y2;
   int64_t ldy2;
   int mirrored;  // not 0: offset k of the map takes the weights of offset kvol - 1 - k
+  int64_t n_in;  // rows of x, 0: not known
 };
 
 // One weight tensor [kvol, cin, cout] on its way to the packed layout [kvol, cout_pad, cin_pad].
@@ -75,6 +76,8 @@ struct ConvOps {
   int (*segment_sum)(hipStream_t s, const void *products, const int32_t *pos, int64_t n_out, int kvol,
                      int64_t seg_rows, int cout, const void *bias, const void *residual, int relu,
                      void *y, const OutPlace *place);
+  // 1 where igemm has the kernel for narrow layers (unsorted, rows of x known)
+  int (*streams)(int kvol, int cin, int cout);
 };
 
 const ConvOps &conv_ops_f16();

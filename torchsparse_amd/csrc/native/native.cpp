@@ -78,6 +78,7 @@ struct Scratch {
     return bytes.data_ptr();
   }
 };
+constexpr int64_t kPadNarrowRows = 131072;
 constexpr int64_t kCounters = 4096;
 std::mutex g_scratch_lock;
 std::map<std::tuple<int, void *, bool>, Scratch> g_scratch;
@@ -183,8 +184,10 @@ Tensor convolve(KernelMap &m, bool transposed, bool backward, const Tensor &x0, 
   tsmi_conv_call c{};
   Tensor x = x0;
   cin = (int)x.size(1);  // (a gradient may come in whole pieces)
-  // (16-bit layers of up to 8 channels have a kernel that takes any number; packed weights are padded already)
-  if (cin * x.element_size() % 16 != 0 && !(x.element_size() == 2 && cin <= 8)) {
+  // (16-bit layers of up to 8 channels have a kernel that takes any number, but over many rows the one for whole
+  // pieces is ahead by more than the copy: 4 -> 32 over 320k rows 52 us, 4 + 23.  Packed weights are padded already.)
+  if (cin * x.element_size() % 16 != 0 &&
+      (x.element_size() != 2 || cin > 8 || (x.size(0) >= kPadNarrowRows && tsmi_conv_streams(m.kvol, 8, cout, dtype_code(x))))) {
     if (pending) check(tsmi_launch_thread_flush());
     x = whole_pieces(x0);
     cin = (int)x.size(1);
@@ -197,6 +200,7 @@ Tensor convolve(KernelMap &m, bool transposed, bool backward, const Tensor &x0, 
   c.residual = residual.defined() ? residual.data_ptr() : nullptr;
   c.relu = relu;
   c.dtype = dtype_code(x);
+  c.n_in = x.size(0);
   c.kvol = m.kvol;
   c.cin = cin;
   c.cout = cout;
@@ -244,6 +248,7 @@ Tensor convolve(KernelMap &m, bool transposed, bool backward, const Tensor &x0, 
     return y;
   }
   if (own_map && m.grouped.defined() && m.kvol == 27 && c.n_out >= rules.group_min_rows && cin > 8 &&
+      !tsmi_conv_streams(m.kvol, cin, cout, c.dtype) &&
       cin * es % 16 == 0 && (cout < 128 || c.n_out >= 65536)) {
     c.grouped = (const int32_t *)m.grouped_at[0];
     c.row_of = (const int32_t *)m.grouped_at[1];
