@@ -693,6 +693,15 @@ const int64_t *tsmi_launch_thread_completed(void);
 int tsmi_launch_thread_flush(void);
 int tsmi_launch_thread_close(void);
 
+/* Gather-GEMM-scatter in two launches: the products of the listed pairs [nnz, cout], rows read through the interleaved
+ * list as they are multiplied (the steps below with a gathered copy in between took 17 us more of 72 for 290k pairs
+ * of 64 channels), then the sums.  Arguments as tsmi_conv_fetch_on_demand's. */
+int tsmi_gs_forward(tsmi_stream_t s, const void *x, const void *w_packed, const int32_t *nbmaps_inter,
+                    int64_t nnz, const int32_t *nbaddrs, const int32_t *qnbaddrs, int64_t qnnz,
+                    const int32_t *row_mask, int64_t n_out, int kvol, int cin, int cout, int dtype,
+                    int transpose, int center_k, const void *bias, const void *residual, int relu,
+                    void *products, void *y);
+
 /* Gather-GEMM-scatter, step 1: buffer[nbaddrs[k] + p, :] = X[in(k,p), :].
  * Replaces gather_all_kernel_pad_sep_with_mask / gather_kernel
  * (convolution/convolution_gather_scatter_cuda.cu:17-40,70-112). */

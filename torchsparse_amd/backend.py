@@ -147,6 +147,8 @@ def _load():
         "tsmi_bn_partial_elems": [_i32],
         "tsmi_bn_backward": [_vp, _vp, _vp, _vp, _i64, _i32, _i32, _i32, _vp, _i32, _vp, _vp, _vp, _vp, _vp,
                              _vp],
+        "tsmi_gs_forward": [_vp, _vp, _vp, _vp, _i64, _vp, _vp, _i64, _vp, _i64, _i32, _i32, _i32, _i32, _i32, _i32,
+                            _vp, _vp, _i32, _vp, _vp],
         "tsmi_gs_gather": [_vp, _vp, _vp, _i64, _i32, _i32, _i32, _vp],
         "tsmi_gs_gemm": [_vp, _vp, _vp, _vp, _vp, _i64, _i64, _i32, _i32, _i32, _i32, _vp],
         "tsmi_gs_scatter": [_vp, _vp, _vp, _vp, _i64, _i32, _i32, _i32, _i32, _vp, _vp, _i32, _vp],
@@ -2847,6 +2849,8 @@ def conv_forward_fetch_on_demand_cuda(in_feats, kernel, nbmaps, sum_nnz, nbaddrs
     planar [2, nnz] list; row_mask is the kmap's output_mask (input_mask when
     transposed) that makes the reduction atomic free."""
     x, wp, (kvol, cin, cout) = _conv_common(in_feats, kernel)
+    x = whole_pieces(x)
+    cin = x.shape[1]
     if row_mask is None:
         raise ValueError("fetch-on-demand needs the kmap's row mask (output_mask / input_mask)")
     y = torch.empty((output_size, cout), dtype=x.dtype, device=x.device)
@@ -2866,11 +2870,13 @@ def conv_forward_gather_scatter_cuda(in_feats, kernel, nbmaps, nbsizes, input_ma
                                      qsum_nnz=None, center_k=-1, bias=None, residual=None,
                                      relu=False) -> torch.Tensor:
     """convolution/convolution_gather_scatter_cuda.cu:279-814: gather -> GEMM per
-    offset -> scatter, here always as three launches over all offsets.  epsilon,
+    offset -> scatter, here always as two launches over all offsets (rows are read as they are multiplied).  epsilon,
     mm_thresh and conv_mode only steer grouping in the reference; results do not
     depend on them and they are accepted and ignored.  nbmaps is the interleaved
     int32 [nnz, 2] list."""
     x, wp, (kvol, cin, cout) = _conv_common(in_feats, kernel)
+    x = whole_pieces(x)
+    cin = x.shape[1]
     nbmaps = _need(nbmaps, torch.int32, "nbmaps")
     nnz = nbmaps.shape[0]
     dev = x.device
@@ -2884,17 +2890,12 @@ def conv_forward_gather_scatter_cuda(in_feats, kernel, nbmaps, nbsizes, input_ma
         qsum_nnz = int(qnbaddrs[-1].item())
     row_mask = input_mask if transpose else output_mask
     code = _dtype_code(x)
-    gathered = torch.empty((max(nnz, 1), cin), dtype=x.dtype, device=dev)
-    products = torch.empty((max(nnz, 1), cout), dtype=x.dtype, device=dev)
-    y = torch.empty((output_size, cout), dtype=x.dtype, device=dev)
-    s = _stream()
-    _check(_C.tsmi_gs_gather(s, _ptr(x), _ptr(nbmaps), nnz, cin, code, int(bool(transpose)),
-                             _ptr(gathered)))
-    _check(_C.tsmi_gs_gemm(s, _ptr(gathered), _ptr(wp), _ptr(nbaddrs), _ptr(qnbaddrs), nnz,
-                           int(qsum_nnz), kvol, cin, cout, code, _ptr(products)))
+    products = x.new_empty(max(nnz, 1), cout)
+    y = x.new_empty(output_size, cout)
     pb, pr = _epilogue_args(bias, residual, x, output_size, cout)
-    _check(_C.tsmi_gs_scatter(s, _ptr(products), _ptr(nbaddrs), _ptr(row_mask), output_size, kvol,
-                              cout, code, center_k, pb, pr, int(relu), _ptr(y)))
+    _check(_C.tsmi_gs_forward(_stream(), _ptr(x), _ptr(wp), _ptr(nbmaps), nnz, _ptr(nbaddrs), _ptr(qnbaddrs),
+                              int(qsum_nnz), _ptr(row_mask), output_size, kvol, cin, cout, code, int(bool(transpose)),
+                              center_k, pb, pr, int(relu), _ptr(products), _ptr(y)))
     return y
 
 

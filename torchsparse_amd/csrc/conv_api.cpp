@@ -230,6 +230,31 @@ extern "C" int tsmi_conv_wgrad_pointwise(tsmi_stream_t s, const void *x, const v
                           workspace_elems, dw);
 }
 
+// Products of the listed pairs, then every output row's sum over its products.
+static int pair_products_and_sums(const char *who, tsmi_stream_t s, const void *x, const void *w_packed,
+                                  const int32_t *rows, int row_step, int64_t nnz, const int32_t *nbaddrs,
+                                  const int32_t *qnbaddrs, int64_t qnnz, const int32_t *row_mask, int64_t n_out,
+                                  int kvol, int cin, int cout, int dtype, int center_k, const void *bias,
+                                  const void *residual, int relu, void *partial, void *y) {
+  const ConvOps *ops = ops_for(dtype);
+  if (int e = check_shapes(who, ops, kvol, cin, cout)) return e;
+  TSMI_REQUIRE(nnz >= 0 && qnnz >= nnz && qnnz % 128 == 0 && n_out >= 0,
+               "%s: bad sizes (nnz %lld, qnnz %lld)", who, (long long)nnz,
+               (long long)qnnz);
+  TSMI_REQUIRE(center_k >= -1 && center_k < kvol, "%s: bad center_k", who);
+  if (n_out == 0) return TSMI_OK;
+  TSMI_REQUIRE(x && w_packed && nbaddrs && qnbaddrs && row_mask && y, "%s: null pointer", who);
+  TSMI_REQUIRE(nnz == 0 || (rows && partial), "%s: null pair list", who);
+  TSMI_REQUIRE(aligned16(x) && aligned16(w_packed) && aligned16(partial),
+               "%s: x, w_packed and partial must be 16-byte aligned", who);
+  if (nnz > 0)
+    if (int e = ops->pairs((hipStream_t)s, x, w_packed, rows, row_step, nbaddrs, qnbaddrs, qnnz, kvol, cin,
+                           cout, partial))
+      return e;
+  return ops->scatter((hipStream_t)s, partial, nbaddrs, row_mask, n_out, kvol, cout, center_k, bias,
+                      residual, relu, y);
+}
+
 extern "C" int tsmi_conv_fetch_on_demand(tsmi_stream_t s, const void *x, const void *w_packed,
                                          const int32_t *nbmaps_planar, int64_t nnz,
                                          const int32_t *nbaddrs, const int32_t *qnbaddrs,
@@ -237,25 +262,19 @@ extern "C" int tsmi_conv_fetch_on_demand(tsmi_stream_t s, const void *x, const v
                                          int kvol, int cin, int cout, int dtype, int transpose,
                                          int center_k, const void *bias, const void *residual,
                                          int relu, void *partial, void *y) {
-  const ConvOps *ops = ops_for(dtype);
-  if (int e = check_shapes("conv_fetch_on_demand", ops, kvol, cin, cout)) return e;
-  TSMI_REQUIRE(nnz >= 0 && qnnz >= nnz && qnnz % 128 == 0 && n_out >= 0,
-               "conv_fetch_on_demand: bad sizes (nnz %lld, qnnz %lld)", (long long)nnz,
-               (long long)qnnz);
-  TSMI_REQUIRE(center_k >= -1 && center_k < kvol, "conv_fetch_on_demand: bad center_k");
-  if (n_out == 0) return TSMI_OK;
-  TSMI_REQUIRE(x && w_packed && nbaddrs && qnbaddrs && row_mask && y,
-               "conv_fetch_on_demand: null pointer");
-  TSMI_REQUIRE(nnz == 0 || (nbmaps_planar && partial), "conv_fetch_on_demand: null pair list");
-  TSMI_REQUIRE(aligned16(x) && aligned16(w_packed) && aligned16(partial),
-               "conv_fetch_on_demand: x, w_packed and partial must be 16-byte aligned");
-  const int32_t *rows = transpose ? nbmaps_planar + nnz : nbmaps_planar;
-  if (nnz > 0)
-    if (int e = ops->pairs((hipStream_t)s, x, w_packed, rows, nbaddrs, qnbaddrs, qnnz, kvol, cin,
-                           cout, partial))
-      return e;
-  return ops->scatter((hipStream_t)s, partial, nbaddrs, row_mask, n_out, kvol, cout, center_k, bias,
-                      residual, relu, y);
+  const int32_t *rows = transpose && nbmaps_planar ? nbmaps_planar + nnz : nbmaps_planar;
+  return pair_products_and_sums("conv_fetch_on_demand", s, x, w_packed, rows, 1, nnz, nbaddrs, qnbaddrs, qnnz,
+                                row_mask, n_out, kvol, cin, cout, dtype, center_k, bias, residual, relu, partial, y);
+}
+
+extern "C" int tsmi_gs_forward(tsmi_stream_t s, const void *x, const void *w_packed, const int32_t *nbmaps_inter,
+                               int64_t nnz, const int32_t *nbaddrs, const int32_t *qnbaddrs, int64_t qnnz,
+                               const int32_t *row_mask, int64_t n_out, int kvol, int cin, int cout, int dtype,
+                               int transpose, int center_k, const void *bias, const void *residual, int relu,
+                               void *products, void *y) {
+  const int32_t *rows = transpose && nbmaps_inter ? nbmaps_inter + 1 : nbmaps_inter;
+  return pair_products_and_sums("gs_forward", s, x, w_packed, rows, 2, nnz, nbaddrs, qnbaddrs, qnnz, row_mask, n_out,
+                                kvol, cin, cout, dtype, center_k, bias, residual, relu, products, y);
 }
 
 extern "C" int tsmi_conv_segments_supported(int kvol, int cin, int cout, int dtype) {
@@ -345,7 +364,7 @@ extern "C" int tsmi_gs_gemm(tsmi_stream_t s, const void *buffer, const void *w_p
   TSMI_REQUIRE(buffer && w_packed && nbaddrs && qnbaddrs && out_buffer, "gs_gemm: null pointer");
   TSMI_REQUIRE(aligned16(buffer) && aligned16(w_packed) && aligned16(out_buffer),
                "gs_gemm: buffers must be 16-byte aligned");
-  return ops->pairs((hipStream_t)s, buffer, w_packed, nullptr, nbaddrs, qnbaddrs, qnnz, kvol, cin,
+  return ops->pairs((hipStream_t)s, buffer, w_packed, nullptr, 1, nbaddrs, qnbaddrs, qnnz, kvol, cin,
                     cout, out_buffer);
 }
 

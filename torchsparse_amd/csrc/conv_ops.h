@@ -46,7 +46,8 @@ struct ConvOps {
                int32_t *counters, int64_t n_counters, const int32_t *order64, const int32_t *order128,
                const OutPlace *place);
   // out[nbaddrs[k] + p, :] = X[rows[nbaddrs[k] + p], :] W[k] over 128-padded pair lists
-  int (*pairs)(hipStream_t s, const void *x, const void *wp, const int32_t *rows,
+  // (row_step entries from one row of `rows` to the next; null: row p is p)
+  int (*pairs)(hipStream_t s, const void *x, const void *wp, const int32_t *rows, int row_step,
                const int32_t *nbaddrs, const int32_t *qnbaddrs, int64_t qnnz, int kvol, int cin,
                int cout, void *out);
   int (*sum_partials)(hipStream_t s, const float *partial, int split, int64_t n_out, int cout,
