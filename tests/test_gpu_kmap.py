@@ -686,3 +686,19 @@ def test_chain_of_strided_levels_from_the_root_rows(name, coords, ks, levels):
             if len(inputs):
                 np.testing.assert_array_equal(host[level, 4:], np.maximum(inputs.max(0), 0))
             inputs = out
+
+
+@pytest.mark.parametrize("n", [32767, 32768, 50001])
+def test_table_and_map_of_many_unordered_rows(n):
+    """Either side of the row count from which keys are stored to their home slots first: every row is found under its
+    own value, and the map is the oracle's."""
+    from torchsparse_amd import backend
+    rng = np.random.default_rng(n)
+    flat = rng.choice(64 * 64 * 20, size=n, replace=False)
+    coords = np.stack([np.zeros(n, np.int64), *np.unravel_index(flat, (64, 64, 20))], 1).astype(np.int32)
+    dev_coords = torch.from_numpy(coords).cuda()
+    table, omap = backend.GPUHashTable.build_subm(dev_coords, (3, 3, 3), 2)
+    assert torch.equal(omap[:n, 13].cpu(), torch.arange(n, dtype=torch.int32))
+    vals = table.vals[table.keys != 0]
+    assert vals.numel() == n and torch.equal(vals.sort()[0].cpu(), torch.arange(1, n + 1, dtype=torch.int32))
+    assert np.array_equal(omap[:n].cpu().numpy(), oracle.kmap_subm(coords, 3)[:n])

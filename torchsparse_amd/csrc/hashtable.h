@@ -63,12 +63,35 @@ __device__ __forceinline__ uint32_t home_slot(const TableView &t, unsigned long 
 // non-empty, so only slots that read as empty (possibly stale) need the atomic.  Distinct
 // keys going into a mostly empty table take the atomic at once and save the round trip.
 template <bool kLoadFirst = true>
-__device__ __forceinline__ uint32_t table_insert(const TableView &t, unsigned long long key,
-                                                 bool *fresh) {
+__device__ __forceinline__ uint32_t table_insert_from(const TableView &t, unsigned long long key, uint32_t slot,
+                                                      bool *fresh) {
   const unsigned long long stored = key + 1;
-  uint32_t slot = home_slot(t, key);
+  if (kLoadFirst) {  // four slots per load, as table_find reads them
+    uint32_t base = slot & ~3u;
+    for (uint32_t probed = 0; probed < t.cap;) {
+      const ulonglong2 lo = *(const ulonglong2 *)(t.keys + base);
+      const ulonglong2 hi = *(const ulonglong2 *)(t.keys + base + 2);
+      const unsigned long long k4[4] = {lo.x, lo.y, hi.x, hi.y};
+      const uint32_t first = slot - base;
+#pragma unroll
+      for (uint32_t j = 0; j < 4; ++j) {
+        if (j < first) continue;
+        unsigned long long prev = k4[j];
+        if (prev == 0ULL) prev = atomicCAS(&t.keys[base + j], 0ULL, stored);
+        if (prev == 0ULL || prev == stored) {
+          *fresh = prev == 0ULL;
+          return base + j;
+        }
+      }
+      probed += 4 - first;
+      base = base + 4 == t.cap ? 0 : base + 4;
+      slot = base;
+    }
+    *fresh = false;
+    return 0xFFFFFFFFu;
+  }
   for (uint32_t probe = 0; probe < t.cap; ++probe) {
-    unsigned long long prev = kLoadFirst ? t.keys[slot] : 0ULL;
+    unsigned long long prev = 0ULL;
     if (prev == 0ULL) prev = atomicCAS(&t.keys[slot], 0ULL, stored);
     if (prev == 0ULL) {
       *fresh = true;
@@ -82,6 +105,11 @@ __device__ __forceinline__ uint32_t table_insert(const TableView &t, unsigned lo
   }
   *fresh = false;
   return 0xFFFFFFFFu;
+}
+
+template <bool kLoadFirst = true>
+__device__ __forceinline__ uint32_t table_insert(const TableView &t, unsigned long long key, bool *fresh) {
+  return table_insert_from<kLoadFirst>(t, key, home_slot(t, key), fresh);
 }
 
 // Returns the slot holding `key` or 0xFFFFFFFF when absent.  A lane reads the four slots of a

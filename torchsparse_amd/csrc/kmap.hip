@@ -70,6 +70,40 @@ __global__ void insert_coords_kernel(TableView t, const int4 *coords, int64_t n,
   t.vals[slot] = (int32_t)(i + 1);
 }
 
+// Many distinct keys into an EMPTY table, two launches: every key is stored to its home slot without asking (one of
+// those that share a home stays, the launch's end makes them visible), then a row whose key is there is done and only
+// the others, a fifth at half load, take compare-and-swaps.  Those run at 6 G/s whatever their addresses - the memory
+// side executes them - and were all of the insert: 160k rows 32 us, 22 in this form.
+__global__ void place_coords_kernel(TableView t, const int4 *coords, int64_t n) {
+  const int64_t i = (int64_t)blockIdx.x * kBlock + threadIdx.x;
+  if (i >= n) return;
+  const int4 c = coords[i];
+  if (!coords_packable(c.x, c.y, c.z, c.w)) return;
+  const unsigned long long key = pack_coords(c.x, c.y, c.z, c.w);
+  t.keys[home_slot(t, key)] = key + 1;
+}
+
+__global__ void settle_coords_kernel(TableView t, const int4 *coords, int64_t n, int32_t *status) {
+  const int64_t i = (int64_t)blockIdx.x * kBlock + threadIdx.x;
+  if (i >= n) return;
+  const int4 c = coords[i];
+  if (!coords_packable(c.x, c.y, c.z, c.w)) {
+    if (status) atomicOr(status, 2);
+    return;
+  }
+  const unsigned long long key = pack_coords(c.x, c.y, c.z, c.w);
+  uint32_t slot = home_slot(t, key);
+  if (t.keys[slot] != key + 1) {
+    bool fresh;
+    slot = table_insert_from<true>(t, key, slot + 1 == t.cap ? 0 : slot + 1, &fresh);
+    if (slot == 0xFFFFFFFFu) {
+      if (status) atomicOr(status, 1);
+      return;
+    }
+  }
+  t.vals[slot] = (int32_t)(i + 1);
+}
+
 // What a submanifold build needs before its insert pass, in one launch: an empty table and a
 // map of -1.  Both are 16-byte stores; thread i takes the i-th int4 of each region it covers.
 __global__ void subm_prepare_kernel(int4 *keys, int64_t keys4, int4 *vals, int64_t vals4, int4 *map,
@@ -1348,6 +1382,18 @@ extern "C" int tsmi_hashtable_clear(tsmi_stream_t s, int64_t *keys, int32_t *val
   return check_launch("tsmi_hashtable_clear");
 }
 
+constexpr int64_t kPlaceRows = 32768;  // (fewer rows are inserted in less than a launch takes)
+
+// Rows into a table that has just been cleared.
+void insert_into_empty(hipStream_t s, const TableView &t, const int4 *coords, int64_t n, int32_t *status) {
+  if (n < kPlaceRows) {
+    hipLaunchKernelGGL(insert_coords_kernel, grid_for(n), dim3(kBlock), 0, s, t, coords, n, status);
+    return;
+  }
+  hipLaunchKernelGGL(place_coords_kernel, grid_for(n), dim3(kBlock), 0, s, t, coords, n);
+  hipLaunchKernelGGL(settle_coords_kernel, grid_for(n), dim3(kBlock), 0, s, t, coords, n, status);
+}
+
 extern "C" int tsmi_hashtable_insert_coords(tsmi_stream_t s, int64_t *keys, int32_t *vals,
                                             int64_t cap, const int32_t *coords, int64_t n,
                                             int32_t *status) {
@@ -1473,9 +1519,7 @@ extern "C" int tsmi_kmap_build_subm(tsmi_stream_t s, int64_t *keys, int32_t *val
   if (odd && !vec_map && cells > 0)
     hipLaunchKernelGGL(fill_kernel<int32_t>, grid_for(cells), dim3(kBlock), 0, (hipStream_t)s,
                        out_in_map, cells, -1);
-  if (n > 0)
-    hipLaunchKernelGGL(insert_coords_kernel, grid_for(n), dim3(kBlock), 0, (hipStream_t)s, t,
-                       (const int4 *)coords, n, status);
+  if (n > 0) insert_into_empty((hipStream_t)s, t, (const int4 *)coords, n, status);
   if (odd) {
     const int64_t total = n * (g.kvol / 2 + 1);
     if (total > 0)
@@ -1492,8 +1536,8 @@ extern "C" int tsmi_coords_check(tsmi_stream_t s, const int32_t *coords, int64_t
   TSMI_REQUIRE(flags && n >= 0 && (n == 0 || coords), "coords_check: bad arguments");
   if (n == 0) return TSMI_OK;
   TSMI_GRID_CHECK(n);
-  hipLaunchKernelGGL(coords_check_kernel, grid_for(n), dim3(kBlock), 0, (hipStream_t)s,
-                     (const int4 *)coords, n, flags);
+  hipLaunchKernelGGL(coords_check_kernel, dim3((unsigned)std::min<int64_t>(256, ceil_div(n, kBlock))), dim3(kBlock), 0,
+                     (hipStream_t)s, (const int4 *)coords, n, flags);
   return check_launch("tsmi_coords_check");
 }
 
