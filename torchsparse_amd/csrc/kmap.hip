@@ -1042,6 +1042,50 @@ __global__ __launch_bounds__(kBlock) void pair_count_kernel(const int32_t *map, 
   }
 }
 
+// One row's KV entries in registers, four per load.
+typedef int map_i32x4 __attribute__((ext_vector_type(4), aligned(4)));
+template <int KV>
+__device__ __forceinline__ void load_map_row(const int32_t *map, int64_t row, int64_t n_rows, int32_t (&m)[KV]) {
+  const int32_t *src = map + min(row, n_rows - 1) * KV;
+#pragma unroll
+  for (int k = 0; k + 4 <= KV; k += 4) {
+    const map_i32x4 q = *(const map_i32x4 *)(src + k);
+#pragma unroll
+    for (int e = 0; e < 4; ++e) m[k + e] = q[e];
+  }
+#pragma unroll
+  for (int k = KV / 4 * 4; k < KV; ++k) m[k] = src[k];
+  if (row >= n_rows) {
+#pragma unroll
+    for (int k = 0; k < KV; ++k) m[k] = -1;
+  }
+}
+
+// pair_count_kernel for a kernel volume known at compile time: no staging, one round trip to memory (a training
+// step's 9 maps over an 80k scan: 103 us, 34).
+template <int KV>
+__global__ __launch_bounds__(kBlock) void pair_count_rows_kernel(const int32_t *map, int64_t n_rows, int64_t nblk,
+                                                                 int32_t *block_counts) {
+  __shared__ int wave_cnt[kBlock / 64][KV];
+  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+  int32_t m[KV];
+  load_map_row<KV>(map, (int64_t)blockIdx.x * kBlock + threadIdx.x, n_rows, m);
+  int my = 0;  // lane k keeps the count of offset k
+#pragma unroll
+  for (int k = 0; k < KV; ++k) {
+    const int c = __popcll(__ballot(m[k] != -1));
+    if (lane == k) my = c;
+  }
+  if (lane < KV) wave_cnt[wave][lane] = my;
+  __syncthreads();
+  if (threadIdx.x < KV) {
+    int c = 0;
+#pragma unroll
+    for (int w = 0; w < kBlock / 64; ++w) c += wave_cnt[w][threadIdx.x];
+    block_counts[(int64_t)threadIdx.x * nblk + blockIdx.x] = c;
+  }
+}
+
 // The pairs of every kernel offset, compacted into that offset's fixed segment, in one launch:
 // in_rows[k * seg_rows + j] = map[row][k] of the j-th pair of offset k, pos[k * n_rows + row] = j
 // (-1 where the row has no pair at k), counts[k] (zero on entry) = pairs of offset k.  A block
@@ -1257,6 +1301,57 @@ __global__ __launch_bounds__(kBlock) void wgrad_pair_fill_kernel(
                   pairs[2 * pos] = v;
                   pairs[2 * pos + 1] = row;
                 });
+}
+
+// wgrad_pair_fill_kernel for a kernel volume known at compile time (the same lists; 9 maps 123 us, 43).
+template <int KV>
+__global__ __launch_bounds__(kBlock) void wgrad_pair_fill_rows_kernel(
+    const int32_t *map, int64_t n_rows, int64_t nblk, const int32_t *offsets, const int32_t *nbsizes, int32_t *pairs,
+    int32_t *seg_steps) {
+  static_assert(KV < 64, "a wavefront scans the lists' sizes");
+  __shared__ int wave_cnt[kBlock / 64][KV];
+  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+  const int64_t row = (int64_t)blockIdx.x * kBlock + threadIdx.x;
+  int32_t m[KV];
+  load_map_row<KV>(map, row, n_rows, m);
+  // lane k: start of offset k's list and this block's place in it
+  const int size = lane < KV ? nbsizes[lane] : 0;
+  const int place = lane < KV ? offsets[(int64_t)lane * nblk + blockIdx.x] : 0;
+  const int padded = (size + kWgradPairStep - 1) / kWgradPairStep * kWgradPairStep;
+  int incl = padded;
+#pragma unroll
+  for (int off = 1; off < 64; off <<= 1) {
+    const int v = __shfl_up(incl, off);
+    if (lane >= off) incl += v;
+  }
+  const int start = incl - padded;
+  if (blockIdx.x == 0) {
+    if (wave == 0 && lane <= KV) seg_steps[lane] = start / kWgradPairStep;
+    for (int k = wave; k < KV; k += kBlock / 64) {  // the padding entries behind each list
+      const int pos = __shfl(start + size, k) + lane;
+      if (pos < __shfl(incl, k)) *(int2 *)(pairs + 2 * (int64_t)pos) = make_int2(-1, -1);
+    }
+  }
+  int my = 0;
+#pragma unroll
+  for (int k = 0; k < KV; ++k) {
+    const int c = __popcll(__ballot(m[k] != -1));
+    if (lane == k) my = c;
+  }
+  if (lane < KV) wave_cnt[wave][lane] = my;
+  __syncthreads();
+  int first = start + place;  // of this wavefront, lane k: in offset k's list
+  if (lane < KV)
+    for (int w = 0; w < wave; ++w) first += wave_cnt[w][lane];
+#pragma unroll
+  for (int k = 0; k < KV; ++k) {
+    const unsigned long long b = __ballot(m[k] != -1);
+    const int base = __shfl(first, k);
+    if (m[k] != -1) {
+      const int64_t pos = base + __popcll(b & ((1ULL << lane) - 1ULL));
+      *(int2 *)(pairs + 2 * pos) = make_int2(m[k], (int32_t)row);
+    }
+  }
 }
 
 // Padded copy of existing interleaved pair lists (offset k's nbsizes[k] pairs follow each
@@ -2054,8 +2149,15 @@ extern "C" int tsmi_pair_lists_count(tsmi_stream_t s, const int32_t *map, int64_
   }
   TSMI_REQUIRE(map && block_counts, "pair_lists_count: null pointer");
   TSMI_REQUIRE(grid_fits(nblk), "pair_lists_count: too many rows");
-  hipLaunchKernelGGL(pair_count_kernel, dim3((unsigned)nblk), dim3(kBlock), 0, (hipStream_t)s, map,
-                     n_rows, kvol, nblk, block_counts);
+  if (kvol == 27)
+    hipLaunchKernelGGL(pair_count_rows_kernel<27>, dim3((unsigned)nblk), dim3(kBlock), 0, (hipStream_t)s, map, n_rows,
+                       nblk, block_counts);
+  else if (kvol == 8)
+    hipLaunchKernelGGL(pair_count_rows_kernel<8>, dim3((unsigned)nblk), dim3(kBlock), 0, (hipStream_t)s, map, n_rows,
+                       nblk, block_counts);
+  else
+    hipLaunchKernelGGL(pair_count_kernel, dim3((unsigned)nblk), dim3(kBlock), 0, (hipStream_t)s, map,
+                       n_rows, kvol, nblk, block_counts);
   hipLaunchKernelGGL(pair_scan_kernel, dim3(kvol), dim3(1024), 0, (hipStream_t)s, block_counts, kvol,
                      nblk, nbsizes);
   return check_launch("tsmi_pair_lists_count");
@@ -2353,8 +2455,15 @@ extern "C" int tsmi_wgrad_pairs_build(tsmi_stream_t s, const int32_t *map, int64
   if (int e = tsmi_pair_lists_count(s, map, n_rows, kvol, block_counts, nbsizes)) return e;
   TSMI_REQUIRE(pairs, "wgrad_pairs_build: null pairs");
   int64_t nblk = ceil_div(n_rows, kBlock);
-  hipLaunchKernelGGL(wgrad_pair_fill_kernel, dim3((unsigned)nblk), dim3(kBlock), 0, (hipStream_t)s,
-                     map, n_rows, kvol, nblk, block_counts, nbsizes, pairs, seg_steps);
+  if (kvol == 27 && (uintptr_t)pairs % 8 == 0)
+    hipLaunchKernelGGL(wgrad_pair_fill_rows_kernel<27>, dim3((unsigned)nblk), dim3(kBlock), 0, (hipStream_t)s, map, n_rows,
+                       nblk, block_counts, nbsizes, pairs, seg_steps);
+  else if (kvol == 8 && (uintptr_t)pairs % 8 == 0)
+    hipLaunchKernelGGL(wgrad_pair_fill_rows_kernel<8>, dim3((unsigned)nblk), dim3(kBlock), 0, (hipStream_t)s, map, n_rows,
+                       nblk, block_counts, nbsizes, pairs, seg_steps);
+  else
+    hipLaunchKernelGGL(wgrad_pair_fill_kernel, dim3((unsigned)nblk), dim3(kBlock), 0, (hipStream_t)s,
+                       map, n_rows, kvol, nblk, block_counts, nbsizes, pairs, seg_steps);
   return check_launch("tsmi_wgrad_pairs_build");
 }
 
