@@ -219,3 +219,25 @@ def test_a_layer_on_its_own(mods, cin, cout, kernel, stride, n, dtype, tol, monk
     one, two, calls = both(stage, step, monkeypatch)
     assert calls == 1
     _close(one, two, tol)
+
+
+def test_layers_given_another_configuration(mods):
+    """A plan made before the layers' dataflow was changed is not used again, nor the lack of one afterwards."""
+    ts, spnn, backbones, _, stage, fuse_inference = mods
+    from torchsparse_amd.nn import functional as F
+    torch.manual_seed(4)
+    coords, feats = cloud(3000, 64, 3), torch.randn(3000, 4, device="cuda", dtype=torch.float16)
+    net = fuse_inference(backbones.SparseResUNet42(in_channels=4).cuda().half().eval())
+
+    def forward():
+        with torch.no_grad():
+            return net(ts.SparseTensor(feats, coords.clone()))[-1].feats.float()
+    want = forward()
+    convs = [m for m in net.modules() if isinstance(m, spnn.Conv3d)]
+    for config in (F.Dataflow.FetchOnDemand, None):
+        for conv in convs:
+            conv._config = None
+            if config is not None:
+                conv._config = F.conv_config.get_default_conv_config().copy()
+                conv._config.dataflow = config
+        assert (forward() - want).norm() / want.norm() < 2e-2

@@ -119,4 +119,6 @@ def fuse_inference(model: nn.Module) -> nn.Module:
         if isinstance(m, nn.Sequential):
             _skip_identities(m)
         m.__dict__.pop("_placed_plan", None)  # (what a network derived from its unfused layers)
+    from . import stage
+    stage.forget()
     return model

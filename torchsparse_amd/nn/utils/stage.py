@@ -26,7 +26,7 @@ from ..functional.conv.conv import kernel_map
 from ..functional.conv.conv_mode import get_conv_mode
 from ..functional.conv.kmap import transpose_kernel_map
 
-__all__ = ["run", "call", "enabled"]
+__all__ = ["run", "call", "enabled", "forget"]
 
 enabled = True  # False: every module is called on its own
 
@@ -38,7 +38,7 @@ class _Unfit(Exception):
 
 
 class _Plan:
-    __slots__ = ("native", "slots", "modules", "members", "training", "cin", "lead", "out_level", "config")
+    __slots__ = ("native", "slots", "modules", "members", "convs", "training", "cin", "lead", "out_level", "config")
 
     def current(self) -> bool:
         """Whether the modules still are what the plan was compiled from: the same parameters and buffers, no hooks."""
@@ -48,6 +48,9 @@ class _Plan:
                 return False
         for table, name, value in self.members:
             if table[name] is not value:
+                return False
+        for conv, config, activation in self.convs:
+            if conv._config is not config or conv.activation != activation:
                 return False
         return True
 
@@ -225,6 +228,7 @@ class _Builder:
         plan.native, plan.training = native, self.training
         plan.slots = tuple((tuple(s[0]), s[1], s[2]) for s in self.slots)
         plan.modules, plan.members = tuple(self.modules), tuple(self.members)
+        plan.convs = tuple((m, m._config, m.activation) for m in self.modules if type(m) is self.Conv3d)
         plan.lead = self.params[0]
         plan.cin = self.ops[0][0][9]
         plan.out_level = self.level
@@ -257,6 +261,11 @@ def _plan_of(owner: nn.Module, modules: Tuple[nn.Module, ...], key) -> Optional[
         if plan is not None and not plan.current():
             return None  # (hooks: the plan waits until they are gone)
     return plan
+
+
+def forget() -> None:
+    """Every plan is made anew: layers were given other configurations, or were fused."""
+    _plans.clear()
 
 
 def _native_map(backend, kmap, transposed: bool):

@@ -31,6 +31,7 @@ from torch import nn
 import torchsparse_amd
 from torchsparse_amd import SparseTensor
 from torchsparse_amd.nn import functional as F
+from torchsparse_amd.nn.utils import stage
 from torchsparse_amd.utils import make_ntuple
 
 __all__ = ["tune"]
@@ -118,6 +119,7 @@ def _set_configs(model: nn.Module, names, overrides: Dict) -> None:
             for k, v in overrides.items():
                 cfg[k] = v
         m._config = cfg
+    stage.forget()  # (whether a run of layers is one stage depends on them)
 
 
 def _time_call(model: nn.Module, inputs, with_backward: bool, runs: int = 2) -> float:
@@ -252,4 +254,5 @@ def tune(model: nn.Module, data_loader: Iterable, n_samples: int = 100,
         for k in _TUNED_KEYS:
             cfg[k] = group_configs[g][k]
         m._config = cfg
+    stage.forget()
     return group_configs
