@@ -221,6 +221,38 @@ def test_a_layer_on_its_own(mods, cin, cout, kernel, stride, n, dtype, tol, monk
     _close(one, two, tol)
 
 
+@pytest.mark.parametrize("dataflow", ["GatherScatter", "FetchOnDemand"])
+@pytest.mark.parametrize("cin,cout,kernel,stride,n,dtype,tol", [
+    (13, 64, 3, 2, 2651, torch.float16, 2e-2), (23, 45, 3, 1, 3000, torch.float32, 2e-5), (32, 32, 2, 2, 515, torch.float32, 2e-5),
+    (64, 128, 3, 1, 5000, torch.bfloat16, 8e-2), (3, 17, 5, 1, 65, torch.float16, 2e-2)])
+def test_training_layers_over_pair_lists(mods, cin, cout, kernel, stride, n, dtype, tol, dataflow, monkeypatch):
+    """A layer, and where it is strided the transposed one back up, in the dataflows of pair lists."""
+    ts, spnn, _, _, stage, _ = mods
+    from torchsparse_amd.nn import functional as F
+    torch.manual_seed(n)
+    config = F.conv_config.get_default_conv_config().copy()
+    config.dataflow = getattr(F.Dataflow, dataflow)
+    coords = cloud(n, max(int((4 * n) ** (1 / 3)), 8), n)
+    layers = [spnn.Conv3d(cin, cout, kernel, stride=stride, padding=kernel // 2 if stride == 1 else 0, config=config)]
+    if stride > 1:
+        layers.append(spnn.Conv3d(cout, cin, kernel, stride=stride, transposed=True, config=config))
+    layers = [m.cuda().to(dtype).train() for m in layers]
+    feats = torch.randn(n, cin, device="cuda").to(dtype)
+
+    def step():
+        x = feats.clone().requires_grad_()
+        y = ts.SparseTensor(x, coords)
+        for m in layers:
+            m.zero_grad(set_to_none=True)
+            y = m(y)
+        y = y.feats
+        y.backward(torch.cos(torch.arange(y.numel(), device="cuda").view_as(y)).to(dtype))
+        return {"y": y.detach(), "dx": x.grad, **{"dw%d" % i: m.kernel.grad for i, m in enumerate(layers)}}
+    one, two, calls = both(stage, step, monkeypatch)
+    assert calls == len(layers)
+    _close(one, two, tol)
+
+
 def test_layers_given_another_configuration(mods):
     """A plan made before the layers' dataflow was changed is not used again, nor the lack of one afterwards."""
     ts, spnn, backbones, _, stage, fuse_inference = mods

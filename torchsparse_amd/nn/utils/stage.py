@@ -9,8 +9,8 @@ kernel maps they need.  A call then fetches or builds the maps - the part that i
 overlaps with what the device is doing - and hands the rest to one native call; in training the stage
 is one autograd node.
 
-``run(module, x)`` answers None for anything a stage does not stand for - hooks on one of the modules, other
-dataflows, mixed types, norms in evaluation mode - and the caller goes through the modules then.  Results are
+``run(module, x)`` answers None for anything a stage does not stand for - hooks on one of the modules, inference in
+the dataflows of pair lists, mixed types, norms in evaluation mode - and the caller goes through the modules then.  Results are
 those of the modules (in training up to the rounding of what no longer goes through memory between them)."""
 import weakref
 from typing import List, Optional, Tuple
@@ -282,6 +282,21 @@ def _native_map(backend, kmap, transposed: bool):
     return handle
 
 
+_LISTS = {_cfg.Dataflow.GatherScatter: 1, _cfg.Dataflow.FetchOnDemand: 2}
+
+
+def _pair_lists(handle, kmap, form: int) -> bool:
+    """Whether the map has the pair lists of that dataflow; the native map has them then, too."""
+    if handle.lists == 0:
+        nbmaps, nnz = kmap["nbmaps"], kmap.get("nnz")
+        if nbmaps is None or nbmaps.dtype != torch.int32 or nbmaps.shape != ((nnz, 2) if form == 1 else (2, nnz)):
+            return False
+        centered = bool(kmap["subm"]) and kmap["out_in_map"].shape[1] % 2 == 1
+        handle.set_lists(form == 2, nbmaps, kmap["nbaddrs"], kmap["qnbaddrs"], int(kmap["qmapsize"]),
+                         kmap["output_mask"], kmap["input_mask"], centered)
+    return handle.lists == form
+
+
 def run(owner: nn.Module, x: SparseTensor, modules: Optional[Tuple[nn.Module, ...]] = None, place=None, also=None):
     """What ``owner`` (or the ``modules`` it stands for, one after the other) makes of ``x``, by one native
     call; None where it has to be called itself.  ``place`` = (buffer, first column): the first convolution's
@@ -309,7 +324,8 @@ def run(owner: nn.Module, x: SparseTensor, modules: Optional[Tuple[nn.Module, ..
     config = plan.config or _cfg.get_global_conv_config()
     if config is None:
         config = _cfg._shared_default_config(get_conv_mode())
-    if config["dataflow"] != _cfg.Dataflow.ImplicitGEMM or config["ifsort"]:
+    lists = config["dataflow"] != _cfg.Dataflow.ImplicitGEMM
+    if config["ifsort"] or (lists and (not training or config["dataflow"] not in _LISTS)):
         return None
     force = config.get("pair_segments")
     caches = x._caches
@@ -330,7 +346,8 @@ def run(owner: nn.Module, x: SparseTensor, modules: Optional[Tuple[nn.Module, ..
             kmap = caches.kmaps.get((fine, kernel_size, stride, dilation))
             if kmap is None or fine not in levels:
                 return None  # (the module's own call raises what there is to raise)
-            transpose_kernel_map(kmap, False)
+            if not lists:
+                transpose_kernel_map(kmap, False)
         else:
             if after != level:
                 strides[after] = tuple(here[a] * stride[a] for a in range(3))
@@ -343,19 +360,23 @@ def run(owner: nn.Module, x: SparseTensor, modules: Optional[Tuple[nn.Module, ..
         if kmap["sizes"][0] == 0 or kmap["sizes"][1] < (2 if training else 1):
             return None
         dict.setdefault(kmap, "kernel_size", kernel_size)
-        handle = _native_map(backend, kmap, transposed)
-        if wide is not None and not transposed:
+        handle = _native_map(backend, kmap, transposed and not lists)
+        if lists and not _pair_lists(handle, kmap, _LISTS[config["dataflow"]]):
+            return None
+        if wide is not None and not transposed and (not lists or kmap["subm"]):
             coarse = levels.get(tuple(2 * s for s in here))
             segments = backend.native_segments(handle, feats, wide, kmap, force, coarse and coarse[0]) or segments
         if uses and not transposed:  # (in training the input gradient of a submanifold layer is a second use)
-            backend.native_grouped(handle, kmap, 2 * uses if training and kmap["subm"] else uses)
+            uses = (0 if lists else uses) + (uses if training and kmap["subm"] else 0)
+            if uses:
+                backend.native_grouped(handle, kmap, uses)
         maps.append(handle)
     out_stride = strides[plan.out_level]
     out_coords, out_range = (x.coords, x.spatial_range) if plan.out_level == 0 else levels[out_stride]
     if training:
         if backend._region_calls:
             backend.flush_launches()
-        y = plan.native.train(feats, maps, segments, backend.group_min_rows)
+        y = plan.native.train(feats, maps, segments, lists, backend.group_min_rows)
         return SparseTensor._make(y, out_coords, out_stride, out_range, caches)
     pending = backend.pending_calls()
     if also is not None:
